@@ -65,6 +65,7 @@ struct GemmArgs {
   int H;
   int skip_i4;             // INT4 token groups belong to the tiled kernel: skip them
   int skip_bf;             // BF16 token groups belong to the tiled kernel: skip them
+  int skip_i8;             // so do the BF16 and INT8 token groups: skip both
 };
 
 // Tiled prefill GEMMs (prefill.hip): work-group tile = 128 expert-sorted rows
@@ -95,14 +96,14 @@ int launch_tile_gemm(int tier, int mode, bool bf, const GemmArgs& a, const float
                      int64_t rs_rows, int64_t x_bytes, int64_t tg_cap, hipStream_t s,
                      int shape = TILE_128x128);
 // The tiles of one projection in one launch (tile_mix_kernel): 128 x 256
-// scaled-operand INT4 tiles over token groups [hdr[1], hdr[3]), 64 x 256 INT4
-// tiles over [hdr[3], hdr[0]) (row sums from launch_group_rowsum), then BF16
-// tiles over [0, hdr[2]).  cap_* bound each range's token groups (0: the range
+// scaled-operand INT4 tiles over token groups [hdr[1], hdr[3]), 128 x 256 INT8
+// tiles over [hdr[2], hdr[1]), 64 x 256 INT4 tiles over [hdr[3], hdr[0]) (row
+// sums from launch_group_rowsum), then BF16 tiles over [0, hdr[2]).  cap_* bound each range's token groups (0: the range
 // is empty); the grid is sized from them and each range's real size is read
 // on the device.
 int launch_tile_mix(int mode, bool bf, const GemmArgs& a, const float* rs, int64_t rs_rows,
-                    int64_t x_bytes, int64_t cap_ps, int64_t cap_64, int64_t cap_bf,
-                    hipStream_t s);
+                    int64_t x_bytes, int64_t cap_ps, int64_t cap_i8, int64_t cap_64,
+                    int64_t cap_bf, hipStream_t s);
 
 // INT4 grouped GEMMs for the shapes outside the tiled / grouped kernels
 // (general.hip): K % 32 == 0, a group size that is a multiple of 32 dividing
@@ -126,6 +127,7 @@ struct RoutePlanParams {
   int tg_cap;
   int i4_group;         // rows per INT4 token group (kTokenGroup or kTokenGroupI4)
   int bf_group;         // rows per BF16 token group (kTokenGroup or kTokenGroupI4)
+  int i8_group;         // rows per INT8 token group (kTokenGroup or kTokenGroupI4)
   // INT4 experts with at least i4_big_rows routed rows (none when 0) take
   // groups of i4_big_group rows and are listed before the other INT4 experts;
   // hdr[3] = the first group of those others (hdr[0] when there are none)

@@ -360,9 +360,9 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TgEntry& te, 
 template <bool BF, int MODE>
 __global__ void __launch_bounds__(NTH, 2) moe_gemm_kernel(GemmArgs a) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[WG_LDS];
-  // Token groups are ordered BF16, INT8, INT4; the BF16 head and the INT4 tail
-  // go to the tiled kernels when those run.
-  const int lo = a.skip_bf ? a.hdr[2] : 0;
+  // Token groups are ordered BF16, INT8, INT4; the BF16 head, the INT8 groups
+  // with it and the INT4 tail go to the tiled kernels when those run.
+  const int lo = a.skip_i8 ? a.hdr[1] : (a.skip_bf ? a.hdr[2] : 0);
   const int n_tg = (a.skip_i4 ? a.hdr[1] : a.hdr[0]) - lo;
   const int U = n_tg * a.n_blocks;
   // XCD-aware order: work-group i runs on XCD i % 8, so each XCD takes a
@@ -577,6 +577,15 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
   const bool tile_bf = tier != nullptr && x32 &&
                        tile_gemm_applies(0, MODE_GATEUP, 2 * I, I, H, gs) &&
                        tile_gemm_applies(0, MODE_DOWN, H, I, I, gs);
+  // INT8 experts take 128 x 256 tiles under the same conditions, with every
+  // BF16 expert of the layer on its tiles too (the grouped kernel then has at
+  // most the INT4 tail of the list left).
+  const bool has_bf = tier != nullptr && b13.bf16 != nullptr;
+  const bool run_i8 = tier != nullptr && b13.i8 != nullptr && x32 && (tile_bf || !has_bf) &&
+                      tile_gemm_applies(1, MODE_GATEUP, 2 * I, I, H, gs) &&
+                      tile_gemm_applies(1, MODE_DOWN, H, I, I, gs) &&
+                      tile_gemm_wide_applies(MODE_GATEUP, 2 * I, I) &&
+                      tile_gemm_wide_applies(MODE_DOWN, H, I);
   // INT4 tile shape, when both projections take the 256-row tiles:
   // * experts averaging fewer than 512 routed rows: 64 sorted rows x 256 weight
   //   rows, the same MFMA work per chunk from fewer bytes of copies and about
@@ -602,6 +611,7 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
   rp.i4_big_rows = !tile ? 0 : (shape == TILE_PS_128x256 ? 1 : (i4_mixed ? kI4BigMinRows : 0));
   rp.i4_big_group = kTokenGroupI4;
   rp.bf_group = tile_bf ? kTokenGroupI4 : kTokenGroup;
+  rp.i8_group = run_i8 ? kTokenGroupI4 : kTokenGroup;
   rp.counters = nullptr;
   rp.n_counters = 0;
   rp.sort_order_out = sort_order_out;
@@ -694,26 +704,32 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
     g.inter = I;
     g.skip_i4 = tile ? 1 : 0;
     g.skip_bf = tile_bf ? 1 : 0;
-    // The grouped kernel runs only for what the tiles leave: INT8 experts, and
-    // INT4 / BF16 experts whose tiled kernel does not apply.  Without a tier
+    g.skip_i8 = run_i8 ? 1 : 0;
+    // The grouped kernel runs only for what the tiles leave: experts of a tier
+    // whose tiled kernel does not apply.  Without a tier
     // array every expert is INT4.  A tile kernel runs only if its tier has
     // experts (an empty launch still costs its grid).
     const bool has_i4 = tier == nullptr || b13.i4 != nullptr;
-    const bool has_bf = tier != nullptr && b13.bf16 != nullptr;
     const bool old_kernel = tier == nullptr ? !tile
-                                            : (b13.i8 != nullptr || (has_i4 && !tile) ||
+                                            : ((b13.i8 != nullptr && !run_i8) || (has_i4 && !tile) ||
                                                (has_bf && !tile_bf));
     const bool run_tile = tile && has_i4, run_tile_bf = tile_bf && has_bf;
-    // INT4 tiles 256 rows wide of both shapes, and BF16 tiles: one launch per
-    // projection (tile_mix_kernel), each range bounded by cap_*
-    const bool mix = run_tile && shape != TILE_128x128 && (run_tile_bf || i4_mixed);
+    // INT4 tiles 256 rows wide of both shapes, INT8 and BF16 tiles: one launch
+    // per projection (tile_mix_kernel), each range bounded by cap_*
+    const bool mix =
+        run_i8 || (run_tile && shape != TILE_128x128 && (run_tile_bf || i4_mixed));
+    const bool rowsum = run_tile && shape != TILE_PS_128x256;  // row-sum tiles run
     const int64_t cap_ps =
-        shape == TILE_PS_128x256
+        !run_tile ? 0
+        : shape == TILE_PS_128x256
             ? L.tg_cap
             : (i4_mixed ? std::min<int64_t>(L.tg_cap, cdiv(L.n, kTokenGroupI4) + L.n / kI4BigMinRows)
                         : 0);
-    const int64_t cap_64 = shape == TILE_64x256 ? L.tg_cap : 0;
-    const int64_t cap_bf = run_tile_bf ? L.tg_cap : 0;
+    // tiers of 128-row groups: at most one partial group per expert
+    const int64_t cap_128 = std::min<int64_t>(L.n, Ep) + cdiv(L.n, kTokenGroupI4);
+    const int64_t cap_64 = run_tile && shape == TILE_64x256 ? L.tg_cap : 0;
+    const int64_t cap_i8 = run_i8 ? cap_128 : 0;
+    const int64_t cap_bf = run_tile_bf ? cap_128 : 0;
     float* rs = reinterpret_cast<float*>(ws + L.rs);
     // gate/up + SiLU: x = hidden, K = H, rows = 2I, out = mid [n, I] (sorted rows)
     g.n_blocks = I / 16;
@@ -732,15 +748,16 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
       st = launch_tile_gemm(0, MODE_GATEUP, bf, g, nullptr, 0, (int64_t)T * H * 2, L.tg_cap, s);
       if (st) return st;
     }
-    if (run_tile) {
-      if (shape != TILE_PS_128x256) {
-        st = launch_group_rowsum(bf, g.x, H, T, H, gs, rs, s);
-        if (st) return st;
-      }
-      st = mix ? launch_tile_mix(MODE_GATEUP, bf, g, rs, T, (int64_t)T * H * 2, cap_ps, cap_64,
-                                 cap_bf, s)
-               : launch_tile_gemm(2, MODE_GATEUP, bf, g, rs, T, (int64_t)T * H * 2, L.tg_cap, s,
-                                  shape);
+    if (rowsum) {
+      st = launch_group_rowsum(bf, g.x, H, T, H, gs, rs, s);
+      if (st) return st;
+    }
+    if (mix) {
+      st = launch_tile_mix(MODE_GATEUP, bf, g, rs, T, (int64_t)T * H * 2, cap_ps, cap_i8, cap_64,
+                           cap_bf, s);
+      if (st) return st;
+    } else if (run_tile) {
+      st = launch_tile_gemm(2, MODE_GATEUP, bf, g, rs, T, (int64_t)T * H * 2, L.tg_cap, s, shape);
       if (st) return st;
     }
     st = record_stage(2, s);
@@ -763,13 +780,15 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
       st = launch_tile_gemm(0, MODE_DOWN, bf, g, nullptr, 0, 0, L.tg_cap, s);
       if (st) return st;
     }
-    if (run_tile) {
-      if (shape != TILE_PS_128x256) {  // sums of the rows the row-sum tiles read
-        st = launch_group_rowsum_tg(bf, g.x, I, I, rp.hdr, rp.tg, L.tg_cap, L.n, rs, s);
-        if (st) return st;
-      }
-      st = mix ? launch_tile_mix(MODE_DOWN, bf, g, rs, L.n, 0, cap_ps, cap_64, cap_bf, s)
-               : launch_tile_gemm(2, MODE_DOWN, bf, g, rs, L.n, 0, L.tg_cap, s, shape);
+    if (rowsum) {  // sums of the rows the row-sum tiles read
+      st = launch_group_rowsum_tg(bf, g.x, I, I, rp.hdr, rp.tg, L.tg_cap, L.n, rs, s);
+      if (st) return st;
+    }
+    if (mix) {
+      st = launch_tile_mix(MODE_DOWN, bf, g, rs, L.n, 0, cap_ps, cap_i8, cap_64, cap_bf, s);
+      if (st) return st;
+    } else if (run_tile) {
+      st = launch_tile_gemm(2, MODE_DOWN, bf, g, rs, L.n, 0, L.tg_cap, s, shape);
       if (st) return st;
     }
   }

@@ -616,6 +616,43 @@ __device__ __forceinline__ int ps_brow(int wn, int t) {
     return wn * 64 + t * 32;
 }
 
+// Store a wave's finished 128 x 64 sub-tile of MFMA 32x32 tiles: accumulator v
+// of tile (mt, t) is row 32 mt + 8 (v / 4) + 4 h + v % 4, column r32 of the
+// tile.  SCALED: column t * 32 + r32 is multiplied by scale[t] first (the INT8
+// row scale of the lane's weight row).
+template <bool BF, int MODE, bool SCALED>
+__device__ __forceinline__ void ps_store(const GemmArgs& a, const TgEntry& te, int nt, int wn,
+                                         int r32, int h, const float (&scale)[2],
+                                         const f32x16_t (&acc)[4][2]) {
+  constexpr int MT = 4, NT = 2, TN = TT;
+  auto val = [&](int mt, int t, int v) { return SCALED ? acc[mt][t][v] * scale[t] : acc[mt][t][v]; };
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int m = mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
+      if (m >= te.cnt) continue;
+      const int pos = te.pos0 + m;
+      if constexpr (MODE == MODE_GATEUP) {
+        uint16_t* mid = reinterpret_cast<uint16_t*>(a.out) + (int64_t)pos * a.out_stride +
+                        nt * (TN / 2) + wn * 32 + r32;
+        *mid = (uint16_t)to_act_bits<BF>(silu_f32(val(mt, 0, v)) * val(mt, 1, v));
+      } else if constexpr (MODE == MODE_PLAIN) {
+        uint16_t* c = reinterpret_cast<uint16_t*>(a.out) + (int64_t)pos * a.out_stride + nt * TN +
+                      wn * 64 + r32;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) c[t * 32] = (uint16_t)to_act_bits<BF>(val(mt, t, v));
+      } else {
+        const int slot = a.row_slot[pos];
+        float* part = reinterpret_cast<float*>(a.out) + (int64_t)slot * a.out_stride + nt * TN +
+                      wn * 64 + r32;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) part[t * 32] = val(mt, t, v);
+      }
+    }
+  }
+}
+
 // Four waves of 128 x 64, two work-groups per CU.  (Eight waves of 128 x 64 in
 // one work-group per CU, each activation chunk feeding 512 weight rows,
 // measured 8 % slower for Mixtral: every chunk's barrier then holds all the
@@ -815,33 +852,157 @@ __device__ __forceinline__ void tile_ps_body(const GemmArgs& a, const TileArgs& 
 #undef EXQ_PS_CHUNK
   wait_vm_all();  // the last (empty) prefetch has drained before the work-group ends
 
-  // Output: accumulator v of tile (mt, t) is row 32 mt + 8 (v / 4) + 4 h + v % 4,
-  // column r32 of the tile.
+  const float one[NT] = {1.f, 1.f};
+  ps_store<BF, MODE, false>(a, te, nt, wn, r32, h, one, acc);
+}
+
+// ---- INT8 experts ------------------------------------------------------------
+// 128 sorted rows x 256 weight rows over the INT8 token groups [hdr[2],
+// hdr[1]), four waves of 128 x 64 (4 x 2 MFMA 32x32x16 tiles) like the
+// scaled-operand INT4 tile, over 64-k chunks of both operands (activations 128
+// rows x 128 B, weights 256 rows x 64 B: 16 KiB each, double buffered).  At
+// k-step s lane half h covers chunk-relative k = 32 h + 8 s + i, so a lane's
+// weight bytes for the chunk are 32 consecutive ones (two ds_read_b128 per
+// weight tile) and its activation fragment is 16 consecutive staged bytes.
+// Every int8 value is exact in bf16 and f16 (|q| <= 128), so the weights are
+// multiplied as signed integers, the fp32 accumulators run over the whole
+// contraction and the row's fp16 scale multiplies the finished sum.
+//
+// Bound: like the INT4 tiles, the activation chunks re-read from L2 for every
+// weight tile beside the matrix pipe (12 VALU instructions per 8 weights and 4
+// MFMAs).  Before, INT8 groups ran on the grouped kernel's 64-row units of 32
+// weight rows, which stage the same activations again for every 32 rows: a
+// mixed OLMoE layer (13 of 64 experts INT8) at 1000 tokens spent 323 + 155 us
+// there.
+template <bool BF>
+__device__ __forceinline__ uint4 deq_i8(uint32_t p0, uint32_t p1) {
+  uint32_t o[4];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int m = mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-      if (m >= cnt) continue;
-      const int pos = pos0 + m;
-      if constexpr (MODE == MODE_GATEUP) {
-        uint16_t* mid = reinterpret_cast<uint16_t*>(a.out) + (int64_t)pos * a.out_stride +
-                        nt * (TN / 2) + wn * 32 + r32;
-        *mid = (uint16_t)to_act_bits<BF>(silu_f32(acc[mt][0][v]) * acc[mt][1][v]);
-      } else if constexpr (MODE == MODE_PLAIN) {
-        uint16_t* c = reinterpret_cast<uint16_t*>(a.out) + (int64_t)pos * a.out_stride + nt * TN +
-                      wn * 64 + r32;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) c[t * 32] = (uint16_t)to_act_bits<BF>(acc[mt][t][v]);
-      } else {
-        const int slot = a.row_slot[pos];
-        float* part = reinterpret_cast<float*>(a.out) + (int64_t)slot * a.out_stride + nt * TN +
-                      wn * 64 + r32;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) part[t * 32] = acc[mt][t][v];
-      }
+  for (int j = 0; j < 4; ++j) {
+    const int p = (int)(j < 2 ? p0 : p1);
+    const int sh = (j & 1) * 16;
+    const float f0 = (float)(int8_t)(p >> sh), f1 = (float)(int8_t)(p >> (sh + 8));
+    if constexpr (BF) {
+      const f32x2_t v = {f0, f1};
+      o[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+    } else {
+      o[j] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(f0, f1));  // exact
     }
   }
+  return uint4{o[0], o[1], o[2], o[3]};
+}
+
+template <bool BF, int MODE>
+__device__ __forceinline__ void tile_i8_body(const GemmArgs& a, const TileArgs& ta, int bid,
+                                             unsigned char* sA0, unsigned char* sA1,
+                                             unsigned char* sB0, unsigned char* sB1) {
+  constexpr int MT = 4, NT = 2, TN = TT;
+  TgEntry te;
+  int nt;
+  if (!tile_unit(a, a.hdr[ta.h_lo], a.hdr[ta.h_hi] - a.hdr[ta.h_lo], ta.n_tiles, bid, te, nt))
+    return;  // INT8 groups [hdr[h_lo], hdr[h_hi])
+  const int cnt = te.cnt, pos0 = te.pos0;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r32 = lane & 31, h = lane >> 5;
+  const int wn = wave;
+  const int K = a.K;
+  const int nch = K / PS_KC;
+  const int widx = a.w.index ? a.w.index[te.e] : te.e;
+  const int64_t ebase = (int64_t)widx * a.n_rows;
+
+  const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.w.i8 + ebase * K, (int64_t)a.n_rows * K);
+  const __amdgpu_buffer_rsrc_t xr =
+      MODE == MODE_GATEUP
+          ? make_rsrc(a.x, ta.x_bytes)
+          : make_rsrc(a.x + (int64_t)pos0 * a.x_stride, (int64_t)cnt * a.x_stride * 2);
+  const __amdgpu_buffer_rsrc_t wnull = make_rsrc(a.w.i8, 0);
+  const __amdgpu_buffer_rsrc_t xnull = make_rsrc(a.x, 0);
+
+  // activations: instruction q fills LDS rows 8j..8j+7 (j = 4 wave + q), 8 columns each;
+  // weights: instruction q fills LDS rows 16j..16j+15, 4 columns each.
+  int voffA[4], voffB[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int m = (wave * 4 + q) * 8 + (lane >> 3);
+    const int xrow = tile_xrow<MODE>(a, te, m);
+    voffA[q] = (MODE == MODE_GATEUP ? xrow : xrow - pos0) * (int)a.x_stride * 2 +
+               ((lane & 7) ^ psa_swz(m)) * 16;
+    const int rho = (wave * 4 + q) * 16 + (lane >> 2);
+    voffB[q] = tile_wrow<MODE, TN>(a, nt, rho) * K + ((lane & 3) ^ psb_swz(rho)) * 16;
+  }
+  const int aoff = r32 * 128 + ((4 * h) ^ psa_swz(r32)) * 16;
+  const int boff = r32 * 64 + ((2 * h) ^ psb_swz(r32)) * 16;  // second half: ^ 16
+  auto prefetch = [&](int st, int ch) {
+    const bool ok = ch < nch;
+    const int chl = ok ? ch : 0;
+    unsigned char* A = st ? sA1 : sA0;
+    unsigned char* B = st ? sB1 : sB0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) dma16(ok ? xr : xnull, A + (wave * 4 + q) * 1024, voffA[q], chl * 128);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) dma16(ok ? wr : wnull, B + (wave * 4 + q) * 1024, voffB[q], chl * 64);
+  };
+
+  f32x16_t acc[MT][NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[mt][t][v] = 0.f;
+
+  // One 64-k chunk, its k-steps software-pipelined as in the scaled-operand tile.
+#define EXQ_I8_CHUNK(ST, PF)                                                                 \
+  do {                                                                                       \
+    const unsigned char* A_ = ST ? sA1 : sA0;                                                \
+    const unsigned char* B_ = ST ? sB1 : sB0;                                                \
+    uint4 bw[NT][2];                                                                         \
+    _Pragma("unroll") for (int t = 0; t < NT; ++t) {                                         \
+      const unsigned char* b_ = B_ + ps_brow<MODE, TN>(wn, t) * 64;                          \
+      bw[t][0] = *reinterpret_cast<const uint4*>(b_ + boff);                                 \
+      bw[t][1] = *reinterpret_cast<const uint4*>(b_ + (boff ^ 16));                          \
+    }                                                                                        \
+    uint4 af[2][MT], wf[2][NT];                                                              \
+    _Pragma("unroll") for (int mt = 0; mt < MT; ++mt)                                        \
+        af[0][mt] = *reinterpret_cast<const uint4*>(A_ + aoff + mt * 32 * 128);              \
+    _Pragma("unroll") for (int t = 0; t < NT; ++t)                                           \
+        wf[0][t] = deq_i8<BF>(bw[t][0].x, bw[t][0].y);                                       \
+    _Pragma("unroll") for (int s = 0; s < 4; ++s) {                                          \
+      const int c_ = s & 1, n_ = c_ ^ 1;                                                     \
+      if (s < 3) {                                                                           \
+        _Pragma("unroll") for (int mt = 0; mt < MT; ++mt)                                    \
+            af[n_][mt] =                                                                     \
+                *reinterpret_cast<const uint4*>(A_ + (aoff ^ ((s + 1) * 16)) + mt * 32 * 128); \
+        _Pragma("unroll") for (int t = 0; t < NT; ++t) {                                     \
+          const uint4 w_ = bw[t][(s + 1) >> 1];                                              \
+          wf[n_][t] = s == 1 ? deq_i8<BF>(w_.x, w_.y) : deq_i8<BF>(w_.z, w_.w);              \
+        }                                                                                    \
+      }                                                                                      \
+      _Pragma("unroll") for (int mt = 0; mt < MT; ++mt)                                      \
+          _Pragma("unroll") for (int t = 0; t < NT; ++t)                                     \
+              acc[mt][t] = mfma32<BF>(af[c_][mt], wf[c_][t], acc[mt][t]);                    \
+      if (s == 0) { PF; }                                                                    \
+      __builtin_amdgcn_sched_barrier(0);                                                     \
+    }                                                                                        \
+  } while (0)
+
+  prefetch(0, 0);
+  for (int ch = 0; ch < nch; ch += 2) {  // nch is even: K is a multiple of 128
+    chunk_barrier();
+    EXQ_I8_CHUNK(0, prefetch(1, ch + 1));
+    chunk_barrier();
+    EXQ_I8_CHUNK(1, prefetch(0, ch + 2));
+  }
+#undef EXQ_I8_CHUNK
+  wait_vm_all();
+
+  float scale[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+    scale[t] = f16_bits_to_f32(
+        a.w.i8_scales[ebase + tile_wrow<MODE, TN>(a, nt, ps_brow<MODE, TN>(wn, t) + r32)]);
+  ps_store<BF, MODE, true>(a, te, nt, wn, r32, h, scale, acc);
 }
 
 // ---- BF16 experts ------------------------------------------------------------
@@ -1089,19 +1250,20 @@ __device__ __forceinline__ int tile_unit_count(int n, int n_tiles) {
   return ((n + 7) >> 3) * 8 * n_tiles;
 }
 
-// The tiles of one projection in one grid, in three ranges whose sizes come
+// The tiles of one projection in one grid, in four ranges whose sizes come
 // from the token-group list on the device: 128 x 256 scaled-operand INT4 tiles
-// over the big-group INT4 experts [hdr[1], hdr[3]), 64 x 256 INT4 tiles over
-// the other INT4 experts [hdr[3], hdr[0]), then BF16 tiles over [0, hdr[2]).
-// All three take 16 KiB per operand stage, so the LDS is shared.  The host
-// sizes the grid from upper bounds; the work-groups past the three ranges
-// return at once, after every real unit in dispatch order.  The longest units
-// (the big experts' 128-row tiles) go first and the BF16 units fill the last,
-// partly empty round of the INT4 ones (DeepSeek-V2-Lite's INT4 gate/up at
-// 2048 tokens is several rounds of the 512 resident work-groups).
+// over the big-group INT4 experts [hdr[1], hdr[3]), 128 x 256 INT8 tiles over
+// [hdr[2], hdr[1]), 64 x 256 INT4 tiles over the other INT4 experts [hdr[3],
+// hdr[0]), then BF16 tiles over [0, hdr[2]).  All take 16 KiB per operand
+// stage, so the LDS is shared.  The host sizes the grid from upper bounds;
+// the work-groups past the four ranges return at once, after every real unit
+// in dispatch order.  The longest units (the 128-row tiles) go first and the
+// BF16 units fill the last, partly empty round of the others
+// (DeepSeek-V2-Lite's INT4 gate/up at 2048 tokens is several rounds of the 512
+// resident work-groups).
 template <bool BF, int MODE>
-__global__ void __launch_bounds__(TT, 2) tile_mix_kernel(GemmArgs a, TileArgs tps, TileArgs t64,
-                                                         TileArgs tbf) {
+__global__ void __launch_bounds__(TT, 2) tile_mix_kernel(GemmArgs a, TileArgs tps, TileArgs ti8,
+                                                         TileArgs t64, TileArgs tbf) {
   static_assert(tile_a_stage<4, 4>() == AB_STAGE && tile_b_stage<4, 4>() == AB_STAGE &&
                     PS_A_STAGE == AB_STAGE && PS_B_STAGE == AB_STAGE,
                 "one LDS layout for the three tiles");
@@ -1116,6 +1278,12 @@ __global__ void __launch_bounds__(TT, 2) tile_mix_kernel(GemmArgs a, TileArgs tp
     return;
   }
   bid -= u_ps;
+  const int u_i8 = tile_unit_count(a.hdr[1] - a.hdr[2], ti8.n_tiles);
+  if (bid < u_i8) {
+    tile_i8_body<BF, MODE>(a, ti8, bid, sA0, sA1, sB0, sB1);
+    return;
+  }
+  bid -= u_i8;
   const int u_64 = tile_unit_count(a.hdr[0] - a.hdr[3], t64.n_tiles);
   if (bid < u_64) {
     tile_gemm_body<BF, MODE, 4, 4>(a, t64, bid, sA0, sA1, sB0, sB1);
@@ -1130,14 +1298,13 @@ __global__ void __launch_bounds__(TT, 2) tile_mix_kernel(GemmArgs a, TileArgs tp
 bool tile_gemm_applies(int tier, int mode, int n_rows, int inter, int K, int group_size) {
   if (K < KC || K % KC != 0 || K > 65536) return false;
   if (tier == 2 && group_size != KC) return false;  // one chunk = one scale group
-  if (tier == 1) return false;
   if (mode == MODE_GATEUP) {
     if (inter % 64 != 0 || n_rows != 2 * inter) return false;
   } else if (n_rows % 128 != 0) {
     return false;
   }
   // 32-bit buffer offsets within one expert's weights
-  if ((int64_t)n_rows * (tier == 2 ? K / 2 : K * 2) > 0x7fffffffLL) return false;
+  if ((int64_t)n_rows * (tier == 2 ? K / 2 : tier == 1 ? K : K * 2) > 0x7fffffffLL) return false;
   return true;
 }
 
@@ -1230,28 +1397,32 @@ int launch_tile_gemm(int tier, int mode, bool bf, const GemmArgs& a, const float
 }
 
 template <int MODE>
-static int launch_mix_mode(bool bf, const GemmArgs& a, const TileArgs& tps, const TileArgs& t64,
-                           const TileArgs& tbf, int64_t grid, hipStream_t s) {
+static int launch_mix_mode(bool bf, const GemmArgs& a, const TileArgs& tps, const TileArgs& ti8,
+                           const TileArgs& t64, const TileArgs& tbf, int64_t grid, hipStream_t s) {
   const dim3 g((unsigned)grid), b(TT);
   if (bf)
-    hipLaunchKernelGGL((tile_mix_kernel<true, MODE>), g, b, 0, s, a, tps, t64, tbf);
+    hipLaunchKernelGGL((tile_mix_kernel<true, MODE>), g, b, 0, s, a, tps, ti8, t64, tbf);
   else
-    hipLaunchKernelGGL((tile_mix_kernel<false, MODE>), g, b, 0, s, a, tps, t64, tbf);
+    hipLaunchKernelGGL((tile_mix_kernel<false, MODE>), g, b, 0, s, a, tps, ti8, t64, tbf);
   return check_launch("tile_mix_kernel");
 }
 
 int launch_tile_mix(int mode, bool bf, const GemmArgs& a, const float* rs, int64_t rs_rows,
-                    int64_t x_bytes, int64_t cap_ps, int64_t cap_64, int64_t cap_bf,
-                    hipStream_t s) {
+                    int64_t x_bytes, int64_t cap_ps, int64_t cap_i8, int64_t cap_64,
+                    int64_t cap_bf, hipStream_t s) {
   if (mode != MODE_GATEUP && mode != MODE_DOWN)
     return set_error(EXQ_ERROR_UNSUPPORTED, "tile_mix: gate/up or down only");
-  TileArgs tps, t64, tbf;
+  TileArgs tps, ti8, t64, tbf;
   tps.rs = nullptr;  // scaled weight operands: no row sums
   tps.rs_rows = 0;
   tps.x_bytes = x_bytes;
   tps.n_tiles = mode == MODE_GATEUP ? a.inter / 128 : a.n_rows / 256;  // 256-row INT4 tiles
   tps.h_lo = 1;
   tps.h_hi = 3;
+  ti8 = tps;
+  ti8.n_tiles = cap_i8 > 0 ? tps.n_tiles : 0;
+  ti8.h_lo = 2;
+  ti8.h_hi = 1;
   t64 = tps;
   t64.rs = rs;
   t64.rs_rows = (int)rs_rows;
@@ -1263,13 +1434,13 @@ int launch_tile_mix(int mode, bool bf, const GemmArgs& a, const float* rs, int64
   tbf.n_tiles = cap_bf > 0 ? (mode == MODE_GATEUP ? a.inter / 64 : a.n_rows / 128) : 0;
   tbf.h_lo = 0;
   tbf.h_hi = 2;
-  const int64_t grid = 8 * cdiv(cap_ps, 8) * tps.n_tiles + 8 * cdiv(cap_64, 8) * t64.n_tiles +
-                       8 * cdiv(cap_bf, 8) * tbf.n_tiles;
+  const int64_t grid = 8 * cdiv(cap_ps, 8) * tps.n_tiles + 8 * cdiv(cap_i8, 8) * ti8.n_tiles +
+                       8 * cdiv(cap_64, 8) * t64.n_tiles + 8 * cdiv(cap_bf, 8) * tbf.n_tiles;
   if (grid <= 0) return EXQ_SUCCESS;
   if (grid > INT32_MAX || rs_rows > INT32_MAX)
     return set_error(EXQ_ERROR_UNSUPPORTED, "tile_mix: problem too large");
-  return mode == MODE_GATEUP ? launch_mix_mode<MODE_GATEUP>(bf, a, tps, t64, tbf, grid, s)
-                             : launch_mix_mode<MODE_DOWN>(bf, a, tps, t64, tbf, grid, s);
+  return mode == MODE_GATEUP ? launch_mix_mode<MODE_GATEUP>(bf, a, tps, ti8, t64, tbf, grid, s)
+                             : launch_mix_mode<MODE_DOWN>(bf, a, tps, ti8, t64, tbf, grid, s);
 }
 
 }  // namespace exq

@@ -469,7 +469,7 @@ __device__ void plan_tail(const RoutePlanParams& p, RouteLds& s) {
   const int gsz = my_cls == 2   ? p.i4_big_group
                   : my_cls == 3 ? p.i4_group
                   : my_cls == 0 ? p.bf_group
-                                : kTokenGroup;
+                                : p.i8_group;
   const int ng = (c + gsz - 1) / gsz;
   int base = 0, first_i4 = 0, first_i8 = 0, first_i4s = 0;
   for (int cl = (p.tier ? 0 : 2); cl <= 3; ++cl) {

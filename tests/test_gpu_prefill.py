@@ -2,8 +2,7 @@
 the GPU vs the fp32 dequantise-then-matmul oracle.  Covers several token
 groups per expert, ragged last groups, one expert taking every row, f16 and
 bf16 activations, the sorted-row GEMM on both kernels (N % 128 == 0 tiles,
-N = 96 does not), group size 256 (the untiled kernel), and mixed tiers where
-BF16 / INT8 groups and INT4 groups run on different kernels in one layer.
+N = 96 does not), group size 256 (the untiled kernel), and mixed tiers.
 Tolerance: relative L2 <= 0.5%."""
 import numpy as np
 import pytest
@@ -209,7 +208,7 @@ def test_prefill_sorted_int4_gemm(N, dtype, device):
 
 @pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
 def test_prefill_mixed_tiers(act, device):
-    """BF16 / INT8 token groups on the grouped kernel, INT4 on the tiled one."""
+    """BF16, INT8 and INT4 token groups on the tiles of one launch."""
     from exq_amd.kernels import MixedExpertBank, fused_experts_mixed
     banner(f"prefill mixed tiers {act}")
     T = 400
@@ -229,8 +228,8 @@ def test_prefill_mixed_tiers(act, device):
 @pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
 def test_prefill_mixed_tiers_large_experts(act, device):
     """A mixed bank with more than 512 rows per routed expert: its INT4
-    experts take the 128 x 256 scaled-operand tiles beside the BF16 tiles and
-    the grouped INT8 kernel."""
+    experts take the 128 x 256 scaled-operand tiles beside the BF16 and INT8
+    tiles."""
     from exq_amd.kernels import MixedExpertBank, fused_experts_mixed
     banner(f"prefill mixed tiers large experts {act}")
     T, E = 1100, 8
@@ -245,6 +244,33 @@ def test_prefill_mixed_tiers_large_experts(act, device):
                               torch.from_numpy(ids).to(device))
     from tests.test_gpu_mixed import _oracle
     assert_close_rel(out, _oracle(bank, x, ids, w), TOL, f"prefill mixed large experts {act}")
+
+
+@pytest.mark.parametrize("H,I,tiers", [
+    (256, 128, [1, 1, 2, 0, 1, 1]),    # one weight tile per group, one 128-k block in the down
+    (768, 384, [1, 2, 1, 1, 1, 0]),    # several tiles, odd 128-k counts
+    (512, 256, [1, 1, 1, 1, 1, 1]),    # no INT4 or BF16 expert beside them
+    (384, 256, [1, 2, 1, 1, 1, 0]),    # H % 256 != 0: the grouped kernel
+])
+@pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
+def test_prefill_int8_tiles(H, I, tiers, act, device):
+    """INT8 experts on the 128 x 256 tiles: experts of 1, 127, 128, 129 and no
+    rows (edges of the 128-row token groups) and one with the rest of the slots."""
+    from exq_amd.kernels import MixedExpertBank, fused_experts_mixed
+    from tests.test_gpu_mixed import _oracle
+    banner(f"prefill int8 tiles H={H} I={I} {act}")
+    T, k, E = 330, 2, len(tiers)
+    w13, w2 = synth.expert_weights_gpu(E, I, H, 990 + H, device)
+    bank = MixedExpertBank.from_weights(w13, w2, tiers, act_dtype=act)
+    counts = [1, 127, 128, 129, 0]
+    flat = np.concatenate([np.full(c, e) for e, c in enumerate(counts)])
+    flat = np.concatenate([flat, np.full(T * k - flat.size, E - 1)])
+    ids = np.random.default_rng(991).permutation(flat).reshape(T, k).astype(np.int64)
+    w = np.random.default_rng(992).random((T, k)).astype(np.float32)
+    x = _hidden(T, H, 993, device, act)
+    out = fused_experts_mixed(x, bank, torch.from_numpy(w).to(device),
+                              torch.from_numpy(ids).to(device))
+    assert_close_rel(out, _oracle(bank, x, ids, w), TOL, f"prefill int8 tiles {H} {I} {act}")
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
