@@ -7,8 +7,10 @@
 namespace exq {
 
 // Tokens of one expert are processed in groups of at most this many rows:
-// four 16-row MFMA tiles on the grouped kernel and on the 64 x 256 INT4 tiles
-// of the prefill kernels, eight on the 128 x 128 tiles.
+// two 16-row MFMA tiles on the rows kernel (rows.hip), four on the grouped
+// kernel and on the 64 x 256 INT4 tiles of the prefill kernels, eight on the
+// 128-row tiles.
+constexpr int kTokenGroupRows = 32;
 constexpr int kTokenGroup = 64;
 constexpr int kTokenGroupI4 = 128;
 // On the 64 x 256 INT4 prefill tiles, an INT4 expert with at least this many
@@ -25,10 +27,11 @@ struct TgEntry {
   int tier;
 };
 
-// Upper bound on the number of token groups for n routed rows over nb experts.
-inline int64_t tg_capacity(int64_t n_rows, int64_t n_buckets) {
+// Upper bound on the number of token groups of (at least) `group` rows for n
+// routed rows over nb experts.
+inline int64_t tg_capacity(int64_t n_rows, int64_t n_buckets, int group = kTokenGroup) {
   int64_t a = n_rows < n_buckets ? n_rows : n_buckets;
-  return a + cdiv(n_rows, kTokenGroup) + 1;
+  return a + cdiv(n_rows, group) + 1;
 }
 
 // Grouped-GEMM modes: gate/up + SiLU into `mid`, plain C = A x W^T, down
@@ -105,12 +108,11 @@ int launch_tile_mix(int mode, bool bf, const GemmArgs& a, const float* rs, int64
                     int64_t x_bytes, int64_t cap_ps, int64_t cap_i8, int64_t cap_64,
                     int64_t cap_bf, hipStream_t s);
 
-// INT4 grouped GEMMs for the shapes outside the tiled / grouped kernels
-// (general.hip): K % 32 == 0, a group size that is a multiple of 32 dividing
-// K, any number of weight rows.  Token groups [hdr[1], hdr[0]) (<= 64 rows),
-// n_blocks = ceil(output columns / 16).
+// INT4 grouped GEMMs over token groups [hdr[1], hdr[0]) of at most
+// kTokenGroupRows rows (rows.hip): K % 32 == 0, a group size that is a multiple
+// of 32 dividing K, any number of weight rows.
 bool general_shape(int64_t K, int64_t group_size);
-int launch_general_gemm(int mode, bool bf, const GemmArgs& a, int64_t tg_cap, hipStream_t s);
+int launch_rows_gemm(int mode, bool bf, const GemmArgs& a, int64_t tg_cap, hipStream_t s);
 
 // Parameters of the routing-plan kernel (one work-group).
 struct RoutePlanParams {

@@ -459,37 +459,56 @@ const hipEvent_t* stage_events() { return g_stage_events_set ? g_stage_events : 
 
 namespace {
 
+// Shapes the decode, tiled and grouped kernels take: H, I and the group size
+// multiples of 128.  Other all-INT4 shapes run on the rows kernels.
+bool standard_shape(const exq_moe_problem* p) {
+  return p->hidden_size % 128 == 0 && p->inter_size % 128 == 0 && p->group_size % 128 == 0;
+}
+
+// Prefill batches of an all-INT4 layer whose experts average at most 32 routed
+// rows run on the rows kernels too (two launches fewer, no row sums, and half
+// the padding of 64-row groups): Qwen3 shape 64 x 256 tiles / rows kernels, us
+// per layer, T = 100 95 / 82, 187 122 / 111, 300 138 / 125, 500 (31 rows) 162 /
+// 161; OLMoE shape T = 187 136 / 115.
+bool rows_shape(const exq_moe_problem* p, bool mixed) {
+  return !standard_shape(p) ||
+         (!mixed && p->n_tokens * p->top_k <= kTokenGroupRows * p->n_experts);
+}
+
 // ---- workspace layout of the fused forward --------------------------------------
 struct FusedLayout {
   size_t sync, hdr, ends, sorted, tg, mid, partial, rs, blk, plan, total;
-  int64_t n, tg_cap;
+  int64_t n, tg_cap, tg_cap_rows;  // tg_cap_rows: the list of the rows kernels
 };
 
-// The decode counters sit at offset 0 with a fixed size, so every fused call
-// finds them at the same place whatever its problem size; each decode launch
+// The decode counters of a decode batch sit at offset 0; each decode launch
 // leaves them zero again.
 FusedLayout fused_layout(const exq_moe_problem& p) {
   FusedLayout L;
   const int64_t kp = p.top_k + p.n_shared;
   const int64_t Ep = p.n_experts + p.n_shared;
   L.n = p.n_tokens * kp;
-  L.tg_cap = tg_capacity(L.n, Ep);
+  const bool dec = decode_path_supported(p.n_tokens, p.top_k, p.n_experts + p.n_shared,
+                                         p.n_shared, p.hidden_size, p.inter_size, p.group_size);
+  L.tg_cap = tg_capacity(L.n, Ep, standard_shape(&p) ? kTokenGroup : kTokenGroupRows);
+  L.tg_cap_rows = tg_capacity(L.n, Ep, kTokenGroupRows);
   size_t off = 0;
-  L.sync = off;     off = align_up(off + kDecodeSyncBytes, 256);
+  L.sync = off;     off = align_up(off + (dec ? kDecodeSyncBytes : 0), 256);
   L.hdr = off;      off = align_up(off + 64, 256);
   L.ends = off;     off = align_up(off + (size_t)(Ep + 1) * 4, 256);
   L.sorted = off;   off = align_up(off + (size_t)L.n * 4, 256);
   L.tg = off;       off = align_up(off + (size_t)L.tg_cap * sizeof(TgEntry), 256);
-  L.mid = off;      off = align_up(off + (size_t)L.n * p.inter_size * 2, 256);
-  // decode batches: one partial set per down k-split
-  const bool dec = decode_path_supported(p.n_tokens, p.top_k, p.n_experts + p.n_shared,
-                                         p.n_shared, p.hidden_size, p.inter_size, p.group_size);
-  L.partial = off;
-  off = align_up(off + (size_t)L.n * p.hidden_size * 4 * (dec ? kDecodeMaxSplit : 1), 256);
-  // group row sums of the tiled prefill kernel: x rows (GATEUP), then mid rows (DOWN)
+  // group row sums of the tiled prefill kernel: x rows (GATEUP), then mid rows
+  // (DOWN).  Right behind the token-group list: the rows kernels' longer list
+  // (standard shapes: I >= 128, so 4 n bytes or more) runs on into it, and they
+  // read no row sums.
   const int64_t rs_x = tile_rowsum_floats(p.n_tokens, p.hidden_size);
   const int64_t rs_mid = tile_rowsum_floats(L.n, p.inter_size);
   L.rs = off;       off = align_up(off + (size_t)(rs_x > rs_mid ? rs_x : rs_mid) * 4, 256);
+  L.mid = off;      off = align_up(off + (size_t)L.n * p.inter_size * 2, 256);
+  // decode batches: one partial set per down k-split
+  L.partial = off;
+  off = align_up(off + (size_t)L.n * p.hidden_size * 4 * (dec ? kDecodeMaxSplit : 1), 256);
   L.blk = off;      off = align_up(off + (size_t)route_plan_blocks(L.n) * Ep * 4, 256);
   L.plan = off;     off = align_up(off + (dec ? decode_plan_bytes(p.n_tokens, p.top_k,
                                                                     p.n_experts, p.n_shared)
@@ -524,12 +543,6 @@ int validate_problem(const exq_moe_problem* p, const char* fn) {
   return EXQ_SUCCESS;
 }
 
-// Shapes the decode, tiled and grouped kernels take: H, I and the group size
-// multiples of 128.  Other all-INT4 shapes run on the general kernels.
-bool standard_shape(const exq_moe_problem* p) {
-  return p->hidden_size % 128 == 0 && p->inter_size % 128 == 0 && p->group_size % 128 == 0;
-}
-
 int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void* topk_ids,
                        const void* topk_weights, const Bank& b13, const Bank& b2,
                        const int8_t* tier, void* out, int64_t* sort_order_out,
@@ -560,18 +573,18 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
   rp.ends = reinterpret_cast<int*>(ws + L.ends);
   rp.sorted = reinterpret_cast<int*>(ws + L.sorted);
   rp.tg = reinterpret_cast<TgEntry*>(ws + L.tg);
-  rp.tg_cap = (int)L.tg_cap;
   // INT4 and BF16 experts run on the tiled kernels (128- or 64-row token
   // groups) when both projections fit them and the gathered activations are 32-bit
   // addressable; INT8 experts (and everything else) on the grouped kernel.
   const int gs = (int)p->group_size;
-  // all-INT4 layers of other shapes: routing plan + general kernels + combine
-  const bool general = !standard_shape(p);
-  EXQ_REQUIRE_SUPPORTED(!general || tier == nullptr,
+  // all-INT4 layers of other shapes or few rows per expert: routing plan + rows
+  // kernels + combine
+  const bool rows = rows_shape(p, tier != nullptr);
+  EXQ_REQUIRE_SUPPORTED(standard_shape(p) || tier == nullptr,
                         "%s: mixed-precision banks need H, I and group_size multiples of 128 "
                         "(got H=%d I=%d g=%d)", fn, H, I, gs);
   const bool x32 = (int64_t)T * H * 2 <= 0x7fffffffLL;
-  const bool tile = !general && x32 && tile_gemm_applies(2, MODE_GATEUP, 2 * I, I, H, gs) &&
+  const bool tile = !rows && x32 && tile_gemm_applies(2, MODE_GATEUP, 2 * I, I, H, gs) &&
                     tile_gemm_applies(2, MODE_DOWN, H, I, I, gs) &&
                     tile_rowsum_floats(L.n, I) * 4 <= 0x7fffffffLL;
   const bool tile_bf = tier != nullptr && x32 &&
@@ -607,7 +620,9 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
   const int shape = !wide_ok ? TILE_128x128
                              : ((int64_t)T * k < 512 * (int64_t)E ? TILE_64x256 : TILE_PS_128x256);
   const bool i4_mixed = shape == TILE_64x256 && T >= kI4BigMinRows;
-  rp.i4_group = tile && shape != TILE_64x256 ? kTokenGroupI4 : kTokenGroup;
+  rp.tg_cap = (int)(rows ? L.tg_cap_rows : L.tg_cap);
+  rp.i4_group = rows ? kTokenGroupRows
+                        : (tile && shape != TILE_64x256 ? kTokenGroupI4 : kTokenGroup);
   rp.i4_big_rows = !tile ? 0 : (shape == TILE_PS_128x256 ? 1 : (i4_mixed ? kI4BigMinRows : 0));
   rp.i4_big_group = kTokenGroupI4;
   rp.bf_group = tile_bf ? kTokenGroupI4 : kTokenGroup;
@@ -622,7 +637,7 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
   struct HookReset {  // the hook is consumed by this call, whatever happens
     ~HookReset() { g_stage_events_set = false; }
   } hook_reset;
-  const bool decode = !general && decode_path_supported(T, k, Ep, p->n_shared, p->hidden_size,
+  const bool decode = standard_shape(p) && decode_path_supported(T, k, Ep, p->n_shared, p->hidden_size,
                                                        p->inter_size, p->group_size);
   int st = EXQ_SUCCESS;
   if (!decode) {
@@ -662,7 +677,7 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
     d.plan = reinterpret_cast<int*>(ws + L.plan);
     d.bf = bf;
     return launch_decode_layer(d, s);  // times its two kernels with the stage events
-  } else if (general) {
+  } else if (rows) {
     GemmArgs g{};
     g.hdr = rp.hdr;
     g.tg = rp.tg;
@@ -671,7 +686,6 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
     g.group_size = gs;
     g.inter = I;
     // gate/up + SiLU -> mid [n, I]; down -> partial [slot, H]
-    g.n_blocks = (int)cdiv(I, 16);
     g.x = reinterpret_cast<const uint16_t*>(hidden);
     g.x_stride = H;
     g.K = H;
@@ -679,11 +693,10 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
     g.n_rows = 2 * I;
     g.out = ws + L.mid;
     g.out_stride = I;
-    st = launch_general_gemm(MODE_GATEUP, bf, g, L.tg_cap, s);
+    st = launch_rows_gemm(MODE_GATEUP, bf, g, rp.tg_cap, s);
     if (st) return st;
     st = record_stage(2, s);
     if (st) return st;
-    g.n_blocks = (int)cdiv(H, 16);
     g.x = reinterpret_cast<const uint16_t*>(ws + L.mid);
     g.x_stride = I;
     g.K = I;
@@ -692,7 +705,7 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
     g.out = ws + L.partial;
     g.out_stride = H;
     g.H = H;
-    st = launch_general_gemm(MODE_DOWN, bf, g, L.tg_cap, s);
+    st = launch_rows_gemm(MODE_DOWN, bf, g, rp.tg_cap, s);
     if (st) return st;
   } else {
     GemmArgs g{};
@@ -816,7 +829,7 @@ int sorted_gemm_impl(const void* a_sorted, int act_dtype, int64_t n_rows, int64_
   EXQ_REQUIRE(n_rows >= 0 && n_rows <= INT32_MAX && n_experts >= 1 && n_experts <= 1024,
               "%s: bad sizes", fn);
   // INT4 weights of other shapes (K % 32, a group size that is a multiple of
-  // 32 dividing K, any N) run on the general kernel; BF16 weights need the
+  // 32 dividing K, any N) run on the rows kernel; BF16 weights need the
   // tiled / grouped kernels' shapes.
   const bool general = tier == 2 && !(K % 128 == 0 && N % 32 == 0 && gs % 128 == 0);
   if (tier == 2) {
@@ -830,7 +843,7 @@ int sorted_gemm_impl(const void* a_sorted, int act_dtype, int64_t n_rows, int64_
     EXQ_REQUIRE_SUPPORTED(N >= 32 && N % 32 == 0, "%s: N=%lld must be a multiple of 32", fn,
                           (long long)N);
   }
-  const int64_t tg_cap = tg_capacity(n_rows, n_experts);
+  const int64_t tg_cap = tg_capacity(n_rows, n_experts, kTokenGroupRows);
   const size_t tg_off = align_up(64, 256);
   const size_t rs_off = tg_off + align_up((size_t)tg_cap * sizeof(TgEntry), 256);
   const size_t need = rs_off + align_up((size_t)tile_rowsum_floats(n_rows, K) * 4, 256);
@@ -849,7 +862,8 @@ int sorted_gemm_impl(const void* a_sorted, int act_dtype, int64_t n_rows, int64_
                     tile_gemm_applies(tier, MODE_PLAIN, (int)N, 0, (int)K, (int)gs) &&
                     tile_rowsum_floats(n_rows, K) * 4 <= 0x7fffffffLL;
   int st = launch_tg_from_ends(ends, (int)n_experts, mask, tier,
-                               tile ? kTokenGroupI4 : kTokenGroup, hdr, tg, (int)tg_cap, s);
+                               general ? kTokenGroupRows : (tile ? kTokenGroupI4 : kTokenGroup), hdr, tg,
+                               (int)tg_cap, s);
   if (st) return st;
   GemmArgs g{};
   g.hdr = hdr;
@@ -863,10 +877,7 @@ int sorted_gemm_impl(const void* a_sorted, int act_dtype, int64_t n_rows, int64_
   g.group_size = (int)gs;
   g.out = c;
   g.out_stride = N;
-  if (general) {
-    g.n_blocks = (int)cdiv(N, 16);
-    return launch_general_gemm(MODE_PLAIN, bf, g, tg_cap, s);
-  }
+  if (general) return launch_rows_gemm(MODE_PLAIN, bf, g, tg_cap, s);
   if (tile && tier == 0) return launch_tile_gemm(0, MODE_PLAIN, bf, g, nullptr, 0, 0, tg_cap, s);
   if (tile) {
     float* rs = reinterpret_cast<float*>(ws + rs_off);
@@ -903,7 +914,8 @@ extern "C" int exq_set_stage_events(void* const* events, int n_events) {
 
 extern "C" size_t exq_moe_gemm_workspace_size(int64_t n_rows, int64_t n_experts, int64_t K) {
   const int64_t r = n_rows > 0 ? n_rows : 0;
-  return align_up(64, 256) + align_up((size_t)tg_capacity(r, n_experts) * sizeof(TgEntry), 256) +
+  return align_up(64, 256) + align_up((size_t)tg_capacity(r, n_experts, kTokenGroupRows) * sizeof(TgEntry),
+                                        256) +
          align_up((size_t)tile_rowsum_floats(r, K > 0 ? K : 0) * 4, 256);
 }
 

@@ -175,7 +175,7 @@ int exq_silu_and_mul(const void* input, int dtype, int64_t rows, int64_t inter,
  * multiple of 32 dividing K (the reference's minimum group is 32,
  * moe_int4_kernel.py:286-290); any N >= 1 (the reference masks the N tail).
  * K, group_size multiples of 128 with N % 32 == 0 take the tiled / grouped
- * kernels, other shapes the general kernel.  exq_moe_gemm_workspace_size
+ * kernels, other shapes the rows kernel.  exq_moe_gemm_workspace_size
  * covers the token-group list and, for INT4 weights with N % 128 == 0 (the
  * tiled kernel), the per-row group sums of A (n_rows * K / 128 floats).
  */
@@ -291,7 +291,7 @@ size_t exq_moe_workspace_size(const exq_moe_problem* problem);
  * combines); larger batches as routing plan + two grouped MFMA GEMMs +
  * combine.  H, I multiples of 32 and a group size that is a multiple of 32
  * dividing both; shapes whose H, I or group size is not a multiple of 128
- * run as routing plan + the general kernels + combine at every batch size
+ * run as routing plan + the rows kernels + combine at every batch size
  * (the mixed-precision layer keeps the 128-multiples).  Replaces the
  * pipeline of _exq_forward_cuda (exq/runtime/sglang_backend.py:65-158:
  * moe_align_block_size -> build_ends_from_slots -> gather_hidden -> GEMM1 ->

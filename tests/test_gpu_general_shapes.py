@@ -2,7 +2,7 @@
 192, contraction lengths below 128 (one group = K, the reference's collapse at
 moe_int4_kernel.py:61-64), and weight-row counts that are not multiples of 32
 (the reference masks the N tail, moe_int4_kernel.py:206-207, 238-240).  Each
-runs the general HIP kernels and is checked against the fp32
+runs the rows kernels and is checked against the fp32
 dequantise-then-matmul oracle; routing arrays bit-exact."""
 import numpy as np
 import pytest
@@ -71,6 +71,36 @@ def test_fused_general_shapes(H, I, g, T, device):
     out16 = fused_experts(x.to(torch.float16), p13, s13, p2, s2, tw, tid)
     assert out16.dtype == torch.float16
     assert_close_rel(out16, ref, TOL, f"fused general fp16 H={H} I={I} g={g} T={T}")
+
+
+@pytest.mark.parametrize("H,I,g", [
+    (2304, 224, 32),    # 72 groups a row: five 16-group scale windows; I not a multiple of 64
+    (1120, 96, 32),     # K % 128 = 96: a short last chunk, windows that straddle chunks
+    (1920, 480, 96),    # groups that straddle 128-k chunks
+    (2176, 320, 64),    # 34 groups: a third window of two
+    (512, 384, 128),    # standard shapes with few rows per expert take the same kernels
+    (1024, 512, 256),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rows_kernel_edges(H, I, g, dtype, device):
+    """Experts with 1, 31, 32, 33 and no rows and one with the rest (edges of the
+    32-row token groups), above 64 tokens."""
+    from exq_amd.kernels import fused_experts
+    banner(f"rows kernel H={H} I={I} g={g} {dtype}")
+    E, T, k = 9, 71, 2
+    p13, s13 = _bank(E, 2 * I, H, g, H + 3 * I, device)
+    p2, s2 = _bank(E, H, I, g, H + 3 * I + 1, device)
+    counts = [1, 31, 32, 33, 0, 2, 16, 17]
+    flat = np.concatenate([np.full(c, e) for e, c in enumerate(counts)])
+    flat = np.concatenate([flat, np.full(T * k - flat.size, E - 1)])
+    rng = np.random.default_rng(H + I)
+    ids = rng.permutation(flat).reshape(T, k).astype(np.int64)
+    w = rng.random((T, k)).astype(np.float32)
+    x = torch.from_numpy(synth.hidden_np(T, H, 4)).to(dtype).to(device)
+    out = fused_experts(x, p13, s13, p2, s2, torch.from_numpy(w).to(device),
+                        torch.from_numpy(ids).to(device))
+    ref = oracle_int4_layer(x, p13, s13, p2, s2, ids, w)
+    assert_close_rel(out, ref, TOL, f"rows kernel H={H} I={I} g={g} {dtype}")
 
 
 def test_general_shape_rejections(device):
