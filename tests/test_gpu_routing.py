@@ -21,8 +21,8 @@ def _ids(T, k, E, seed, dtype=torch.int64, invalid=0):
 
 CASES = [(1, 8, 64), (16, 8, 64), (64, 8, 128), (5, 2, 8), (1, 1, 1), (4096, 2, 8),
          (2048, 6, 64), (300, 8, 1000)]
-# above 2048 items or 1023 experts: the multi-block sort (several work-groups,
-# each recounting every item); up to 4095 experts
+# many items, or so many experts that the multi-block sort runs (several
+# work-groups, each recounting every item); up to 4095 experts
 WIDE = [(2048, 8, 64), (4096, 8, 128), (64, 8, 3000), (333, 8, 4095), (9000, 2, 1500),
         (257, 8, 8)]
 
@@ -42,6 +42,28 @@ def test_dispatch_bit_exact(T, k, E, dtype, device):
     assert np.array_equal(so.cpu().numpy(), r_so)
     assert np.array_equal(si.cpu().numpy(), r_si)
     assert np.array_equal(ends.cpu().numpy(), r_ends)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 2048, 2049, 4096, 4097, 16385])
+@pytest.mark.parametrize("E", [1, 2, 127, 128, 511])
+def test_sort_segment_and_bucket_edges(n, E, device):
+    """One work-group sort (64-item segments, at most 4,096 items and 32,768
+    (segment, bucket) counts) and the multi-block sort past those limits, with
+    skewed ids, out-of-range ones and one bucket holding almost everything."""
+    from exq_amd.kernels.exq_dispatch import dispatch
+    banner(f"sort edges n={n} E={E}")
+    rng = np.random.default_rng(n * 7 + E)
+    ids = np.minimum(rng.geometric(0.3, n) - 2, E + 1).astype(np.int64)  # -1 .. E + 1
+    ids[rng.random(n) < 0.1] = rng.integers(0, E)
+    so = torch.empty(n, dtype=torch.int64, device=device)
+    si = torch.empty(n, dtype=torch.int64, device=device)
+    ends = torch.empty(E + 1, dtype=torch.int32, device=device)
+    dispatch(torch.from_numpy(ids).to(device), so, si, ends, E)
+    key = np.where((ids >= 0) & (ids < E), ids, E)
+    order = np.argsort(key, kind="stable")
+    assert np.array_equal(so.cpu().numpy(), order)
+    assert np.array_equal(si.cpu().numpy(), ids[order])
+    assert np.array_equal(ends.cpu().numpy(), np.searchsorted(key[order], np.arange(E + 1)))
 
 
 @pytest.mark.parametrize("T,k,E", CASES[:6] + [(2048, 8, 64), (64, 8, 2000), (600, 4, 1100)])
