@@ -2,6 +2,8 @@
 // libexq_hip.so.  Not part of the C ABI.
 #pragma once
 
+#include <type_traits>
+
 #include "exq_common.h"
 
 namespace exq {
@@ -202,6 +204,17 @@ size_t decode_plan_bytes(int64_t T, int64_t k, int64_t E, int64_t n_shared);
 bool decode_path_supported(int64_t T, int64_t k, int64_t Ep, int64_t n_shared, int64_t H,
                            int64_t I, int64_t group_size);
 int launch_decode_layer(const DecodeLaunch& d, hipStream_t s);
+
+// f(dtype constant) for a float dtype code.
+template <typename F>
+void with_dtype(int dtype, F f) {
+  if (dtype == EXQ_DTYPE_F32)
+    f(std::integral_constant<int, EXQ_DTYPE_F32>{});
+  else if (dtype == EXQ_DTYPE_BF16)
+    f(std::integral_constant<int, EXQ_DTYPE_BF16>{});
+  else
+    f(std::integral_constant<int, EXQ_DTYPE_F16>{});
+}
 
 // The four stage events installed with exq_set_stage_events for the current
 // call on this thread, or nullptr.
