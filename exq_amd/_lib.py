@@ -62,6 +62,10 @@ _SIGNATURES = {
     "exq_moe_gemm_workspace_size": ([_I64, _I64, _I64], _SZ),
     "exq_moe_int4_gemm": ([_P, _INT, _I64, _I64, _P, _P, _I64, _I64, _I64, _P, _P, _P, _SZ, _P], _INT),
     "exq_moe_grouped_gemm": ([_P, _INT, _I64, _I64, _P, _I64, _I64, _P, _P, _P, _P, _SZ, _P], _INT),
+    "exq_moe_routed_gemm_workspace_size": ([_I64, _I64, _I64, _I64], _SZ),
+    "exq_moe_routed_gemm": ([_P, _INT, _I64, _I64, _P, _INT, _I64, _P, _P, _P, _I64, _I64, _I64, _P, _P, _P, _SZ, _P], _INT),
+    "exq_unsort_combine_workspace_size": ([_I64, _I64, _I64], _SZ),
+    "exq_unsort_combine": ([_P, _INT, _P, _INT, _P, _INT, _I64, _I64, _I64, _I64, _P, _P, _SZ, _P], _INT),
     "exq_moe_workspace_size": ([C.POINTER(MoeProblem)], _SZ),
     "exq_moe_int4_fused_forward": ([C.POINTER(MoeProblem), _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P], _INT),
     "exq_moe_mixed_forward": ([C.POINTER(MoeProblem), _P, _P, _P, C.POINTER(ExpertBank), _P, _P, _P, _P, _SZ, _P], _INT),

@@ -257,6 +257,32 @@ extern "C" int exq_gather_hidden(const void* hidden, int dtype, int64_t n_tokens
   return check_launch("gather_rows_kernel");
 }
 
+namespace exq {
+
+// result[t] = sum_j w[t, j] * down[inv[t * k + j]] (combine_kernel).
+static int launch_combine(const void* down_out, int dtype, const int32_t* inv, int64_t n_active,
+                          const void* router_weights, int weights_dtype, int64_t n_tokens,
+                          int64_t top_k, int64_t hidden_size, void* result, hipStream_t s) {
+  const bool vec = hidden_size % 8 == 0 && ((uintptr_t)down_out | (uintptr_t)result) % 16 == 0;
+  const int64_t units = n_tokens * (hidden_size / (vec ? 8 : 1));
+  EXQ_REQUIRE(cdiv(units, 256) <= INT32_MAX, "combine: too many outputs");
+  const dim3 grid((unsigned)cdiv(units, 256));
+  with_dtype(dtype, [&](auto dt) {
+    constexpr int DT = decltype(dt)::value;
+    if (vec)
+      hipLaunchKernelGGL((combine_kernel<DT, 8>), grid, dim3(256), 0, s, down_out, inv,
+                         router_weights, weights_dtype, units, (int)top_k, (int)hidden_size,
+                         (int)n_active, result);
+    else
+      hipLaunchKernelGGL((combine_kernel<DT, 1>), grid, dim3(256), 0, s, down_out, inv,
+                         router_weights, weights_dtype, units, (int)top_k, (int)hidden_size,
+                         (int)n_active, result);
+  });
+  return check_launch("combine_kernel");
+}
+
+}  // namespace exq
+
 extern "C" size_t exq_combine_workspace_size(int64_t n_active) {
   return align_up((size_t)(n_active > 0 ? n_active : 0) * sizeof(int32_t), 256);
 }
@@ -285,22 +311,74 @@ extern "C" int exq_combine(const void* down_out, int dtype, const int64_t* sort_
                      sort_order, (int)n_active, inv);
   int st = check_launch("inverse_perm_kernel");
   if (st) return st;
-  const bool vec = hidden_size % 8 == 0 && ((uintptr_t)down_out | (uintptr_t)result) % 16 == 0;
-  const int64_t units = n_tokens * (hidden_size / (vec ? 8 : 1));
-  EXQ_REQUIRE(cdiv(units, 256) <= INT32_MAX, "exq_combine: too many outputs");
-  const dim3 grid((unsigned)cdiv(units, 256));
-  with_dtype(dtype, [&](auto dt) {
-    constexpr int DT = decltype(dt)::value;
-    if (vec)
-      hipLaunchKernelGGL((combine_kernel<DT, 8>), grid, dim3(256), 0, s, down_out, inv,
-                         router_weights, weights_dtype, units, (int)top_k, (int)hidden_size,
-                         (int)n_active, result);
-    else
-      hipLaunchKernelGGL((combine_kernel<DT, 1>), grid, dim3(256), 0, s, down_out, inv,
-                         router_weights, weights_dtype, units, (int)top_k, (int)hidden_size,
-                         (int)n_active, result);
-  });
-  return check_launch("combine_kernel");
+  return launch_combine(down_out, dtype, inv, n_active, router_weights, weights_dtype, n_tokens,
+                        top_k, hidden_size, result, s);
+}
+
+namespace {
+// Workspace of exq_unsort_combine: inverse positions, then (only when the sort
+// does not fit one work-group) sort order, sorted ids and boundaries.
+struct UnsortLayout {
+  size_t order, ids, ends, total;
+};
+UnsortLayout unsort_layout(int64_t n, int64_t n_experts) {
+  UnsortLayout L;
+  const bool one = inverse_sort_fits(n, n_experts + 1);
+  size_t off = align_up((size_t)(n > 0 ? n : 0) * 4, 256);
+  L.order = off;  off += one ? 0 : align_up((size_t)n * 8, 256);
+  L.ids = off;    off += one ? 0 : align_up((size_t)n * 8, 256);
+  L.ends = off;   off += one ? 0 : align_up((size_t)(n_experts + 1) * 4, 256);
+  L.total = off;
+  return L;
+}
+}  // namespace
+
+extern "C" size_t exq_unsort_combine_workspace_size(int64_t n_tokens, int64_t top_k,
+                                                    int64_t n_experts) {
+  return unsort_layout(n_tokens * top_k, n_experts).total;
+}
+
+extern "C" int exq_unsort_combine(const void* sorted_rows, int dtype, const void* router_indices,
+                                  int ids_dtype, const void* router_weights, int weights_dtype,
+                                  int64_t n_tokens, int64_t top_k, int64_t n_experts,
+                                  int64_t hidden_size, void* result, void* workspace,
+                                  size_t workspace_bytes, exq_stream stream) {
+  const char* fn = "exq_unsort_combine";
+  EXQ_REQUIRE(is_float_dtype(dtype) && is_float_dtype(weights_dtype),
+              "%s: dtypes must be f32, f16 or bf16", fn);
+  EXQ_REQUIRE(is_index_dtype(ids_dtype), "%s: ids must be i32 or i64", fn);
+  EXQ_REQUIRE(top_k >= 1 && n_tokens >= 0 && n_tokens * top_k <= INT32_MAX && hidden_size > 0 &&
+                  n_experts >= 1 && n_experts < 4096,
+              "%s: bad sizes", fn);
+  EXQ_REQUIRE(cdiv(hidden_size, 256) <= 65535, "%s: hidden_size=%lld too large", fn,
+              (long long)hidden_size);
+  if (n_tokens == 0) return EXQ_SUCCESS;
+  const int64_t n = n_tokens * top_k;
+  const UnsortLayout L = unsort_layout(n, n_experts);
+  if (workspace_bytes < L.total)
+    return set_error(EXQ_ERROR_WORKSPACE_TOO_SMALL, "%s: workspace %zu < %zu bytes", fn,
+                     workspace_bytes, L.total);
+  EXQ_REQUIRE(sorted_rows && router_indices && router_weights && result && workspace,
+              "%s: null pointer", fn);
+  hipStream_t s = as_stream(stream);
+  unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
+  int32_t* inv = reinterpret_cast<int32_t*>(ws);
+  int st;
+  if (inverse_sort_fits(n, n_experts + 1)) {
+    st = launch_inverse_sort(router_indices, ids_dtype, (int)n, (int)n_experts, inv, s);
+  } else {
+    int64_t* order = reinterpret_cast<int64_t*>(ws + L.order);
+    st = exq_dispatch(router_indices, ids_dtype, n, n_experts, order,
+                      reinterpret_cast<int64_t*>(ws + L.ids),
+                      reinterpret_cast<int32_t*>(ws + L.ends), stream);
+    if (st) return st;
+    hipLaunchKernelGGL(inverse_perm_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, s, order,
+                       (int)n, inv);
+    st = check_launch("inverse_perm_kernel");
+  }
+  if (st) return st;
+  return launch_combine(sorted_rows, dtype, inv, n, router_weights, weights_dtype, n_tokens,
+                        top_k, hidden_size, result, s);
 }
 
 extern "C" int exq_silu_and_mul(const void* input, int dtype, int64_t rows, int64_t inter,

@@ -59,6 +59,7 @@ struct GemmArgs {
   const uint16_t* x;       // activations (f16/bf16 bits)
   int64_t x_stride;        // elements per activation row
   const int* row_slot;     // expert-sorted position -> slot (GATEUP input, DOWN output)
+  int gather;              // PLAIN: rows of x are tokens too (row_slot / slot_div), as in GATEUP
   int slot_div;            // slots per token (kp)
   int K;                   // contraction length, multiple of 128
   Bank w;
@@ -115,6 +116,9 @@ int launch_tile_mix(int mode, bool bf, const GemmArgs& a, const float* rs, int64
 // of 32 dividing K, any number of weight rows.
 bool general_shape(int64_t K, int64_t group_size);
 int launch_rows_gemm(int mode, bool bf, const GemmArgs& a, int64_t tg_cap, hipStream_t s);
+// The same for unquantised weights, plain C = A x W^T over the BF16 token groups
+// [0, hdr[2]): K % 128 == 0, any number of weight rows.
+int launch_rows_gemm_bf16(bool bf, const GemmArgs& a, int64_t tg_cap, hipStream_t s);
 
 // Parameters of the routing-plan kernel (one work-group).
 struct RoutePlanParams {
@@ -122,7 +126,9 @@ struct RoutePlanParams {
   int ids_dtype;
   int T, k, kp, E, Ep;  // kp = k + n_shared, Ep = E + n_shared
   int n;                // T * kp
-  const int8_t* tier;   // [Ep] or null (all INT4)
+  const int8_t* tier;   // [Ep] or null (all of tier all_tier)
+  int all_tier;
+  const int32_t* mask;  // [Ep] or null: experts whose entry is 0 get no token groups
   int* hdr;             // [0] token groups, [1] first INT4 group, [2] first INT8 group,
                         // [3] first INT4 group of an expert below i4_big_rows
   int* ends;            // [Ep + 1]
@@ -151,6 +157,13 @@ struct RoutePlanParams {
 constexpr int kRoutePlanOneBlock = 2048;
 int64_t route_plan_blocks(int64_t n);
 int launch_route_plan(const RoutePlanParams& p, hipStream_t stream);
+
+// The stable sort of n ids over n_experts (ids outside last, as exq_dispatch) as
+// inverse positions, inv[i] = place of id i, when one work-group takes it
+// (nb = n_experts + 1 buckets).
+bool inverse_sort_fits(int64_t n, int64_t nb);
+int launch_inverse_sort(const void* ids, int ids_dtype, int n, int E, int32_t* inv,
+                        hipStream_t stream);
 
 // Token groups from user-provided expert boundaries (sorted-row GEMM API).
 int launch_tg_from_ends(const int32_t* ends, int E, const int32_t* expert_mask, int tier,

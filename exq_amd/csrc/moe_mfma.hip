@@ -4,7 +4,7 @@
 // Work decomposition.  A token group (TgEntry: one expert, <= 64 expert-sorted
 // rows) times a block of weight rows is one work-group unit:
 //   GATEUP: 16 gate rows j and the 16 matching up rows I + j  (SiLU fused)
-//   PLAIN / DOWN: 32 consecutive weight rows
+//   DOWN: 32 consecutive weight rows
 // The four waves of a work-group split the contraction (K) into 128-element
 // k-blocks; their fp32 partial tiles are summed through LDS at the end.
 //
@@ -342,10 +342,6 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TgEntry& te, 
         uint16_t* mid = reinterpret_cast<uint16_t*>(a.out);
         mid[(int64_t)pos * a.out_stride + blk * 16 + r16] =
             (uint16_t)to_act_bits<BF>(silu_f32(g0) * g1);
-      } else if constexpr (MODE == MODE_PLAIN) {
-        uint16_t* c = reinterpret_cast<uint16_t*>(a.out);
-        c[(int64_t)pos * a.out_stride + rows[0]] = (uint16_t)to_act_bits<BF>(g0);
-        c[(int64_t)pos * a.out_stride + rows[1]] = (uint16_t)to_act_bits<BF>(g1);
       } else {
         float* part = reinterpret_cast<float*>(a.out);
         const int slot = a.row_slot[pos];
@@ -475,6 +471,10 @@ bool rows_shape(const exq_moe_problem* p, bool mixed) {
          (!mixed && p->n_tokens * p->top_k <= kTokenGroupRows * p->n_experts);
 }
 
+// The unquantised GEMM takes the rows kernel up to this many rows per expert on
+// average.
+constexpr int64_t kRowsBf16Max = 32;
+
 // ---- workspace layout of the fused forward --------------------------------------
 struct FusedLayout {
   size_t sync, hdr, ends, sorted, tg, mid, partial, rs, blk, plan, total;
@@ -569,6 +569,8 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
   rp.T = T; rp.k = k; rp.kp = kp; rp.E = E; rp.Ep = Ep;
   rp.n = (int)L.n;
   rp.tier = tier;
+  rp.all_tier = 2;
+  rp.mask = nullptr;
   rp.hdr = reinterpret_cast<int*>(ws + L.hdr);
   rp.ends = reinterpret_cast<int*>(ws + L.ends);
   rp.sorted = reinterpret_cast<int*>(ws + L.sorted);
@@ -821,18 +823,53 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
   return record_stage(3, s);
 }
 
-int sorted_gemm_impl(const void* a_sorted, int act_dtype, int64_t n_rows, int64_t K,
-                     const Bank& bank, int tier, int64_t n_experts, int64_t N, int64_t gs,
-                     const int32_t* ends, const int32_t* mask, void* c, void* workspace,
-                     size_t workspace_bytes, hipStream_t s, const char* fn) {
-  EXQ_REQUIRE(is_act_dtype(act_dtype), "%s: act dtype must be f16 or bf16", fn);
-  EXQ_REQUIRE(n_rows >= 0 && n_rows <= INT32_MAX && n_experts >= 1 && n_experts <= 1024,
-              "%s: bad sizes", fn);
+// Sorted-row grouped GEMM C = A x W^T of one tier (2 INT4, 0 unquantised), from
+// expert boundaries (`ends`, rows already sorted) or from the routing itself
+// (`ids`: rows of A are tokens, gathered by the GEMM).
+struct SortedGemm {
+  const void* a;
+  int act_dtype;
+  int64_t n_rows;  // expert-sorted rows
+  int64_t K, E, N, gs;
+  Bank bank;
+  int tier;
+  const int32_t* mask;
+  void* c;
+  const int32_t* ends;
+  const void* ids;  // routed: [n_tokens, top_k]
+  int ids_dtype;
+  int64_t n_tokens, top_k;
+};
+
+struct SortedLayout {
+  size_t tg, rs, ends, sorted, blk, total;
+  int64_t tg_cap;
+};
+
+SortedLayout sorted_layout(int64_t n_rows, int64_t rs_rows, int64_t E, int64_t K, bool routed) {
+  SortedLayout L;
+  L.tg_cap = tg_capacity(n_rows, E, kTokenGroupRows);
+  size_t off = align_up(64, 256);  // hdr
+  L.tg = off;      off += align_up((size_t)L.tg_cap * sizeof(TgEntry), 256);
+  L.rs = off;      off += align_up((size_t)tile_rowsum_floats(rs_rows, K) * 4, 256);
+  L.ends = off;    off += routed ? align_up((size_t)(E + 1) * 4, 256) : 0;
+  L.sorted = off;  off += routed ? align_up((size_t)n_rows * 4, 256) : 0;
+  L.blk = off;     off += routed ? align_up((size_t)route_plan_blocks(n_rows) * E * 4, 256) : 0;
+  L.total = off;
+  return L;
+}
+
+int sorted_gemm_impl(const SortedGemm& p, void* workspace, size_t workspace_bytes, hipStream_t s,
+                     const char* fn) {
+  const int64_t K = p.K, N = p.N, gs = p.gs, n_rows = p.n_rows;
+  const bool routed = p.ids != nullptr;
+  EXQ_REQUIRE(is_act_dtype(p.act_dtype), "%s: act dtype must be f16 or bf16", fn);
+  EXQ_REQUIRE(n_rows >= 0 && n_rows <= INT32_MAX && p.E >= 1 && p.E <= 1024, "%s: bad sizes", fn);
   // INT4 weights of other shapes (K % 32, a group size that is a multiple of
   // 32 dividing K, any N) run on the rows kernel; BF16 weights need the
   // tiled / grouped kernels' shapes.
-  const bool general = tier == 2 && !(K % 128 == 0 && N % 32 == 0 && gs % 128 == 0);
-  if (tier == 2) {
+  const bool general = p.tier == 2 && !(K % 128 == 0 && N % 32 == 0 && gs % 128 == 0);
+  if (p.tier == 2) {
     EXQ_REQUIRE_SUPPORTED(general_shape(K, gs),
                           "%s: K=%lld and group_size=%lld: the group size must be a multiple "
                           "of 32 dividing K", fn, (long long)K, (long long)gs);
@@ -843,49 +880,81 @@ int sorted_gemm_impl(const void* a_sorted, int act_dtype, int64_t n_rows, int64_
     EXQ_REQUIRE_SUPPORTED(N >= 32 && N % 32 == 0, "%s: N=%lld must be a multiple of 32", fn,
                           (long long)N);
   }
-  const int64_t tg_cap = tg_capacity(n_rows, n_experts, kTokenGroupRows);
-  const size_t tg_off = align_up(64, 256);
-  const size_t rs_off = tg_off + align_up((size_t)tg_cap * sizeof(TgEntry), 256);
-  const size_t need = rs_off + align_up((size_t)tile_rowsum_floats(n_rows, K) * 4, 256);
+  const int64_t rs_rows = routed ? p.n_tokens : n_rows;  // rows of A
+  const SortedLayout L = sorted_layout(n_rows, rs_rows, p.E, K, routed);
   if (n_rows == 0) return EXQ_SUCCESS;
-  if (workspace_bytes < need)
+  if (workspace_bytes < L.total)
     return set_error(EXQ_ERROR_WORKSPACE_TOO_SMALL, "%s: workspace %zu < %zu bytes", fn,
-                     workspace_bytes, need);
-  EXQ_REQUIRE(a_sorted && c && ends && workspace, "%s: null pointer", fn);
-  EXQ_REQUIRE(((uintptr_t)a_sorted | (uintptr_t)workspace) % 16 == 0,
+                     workspace_bytes, L.total);
+  EXQ_REQUIRE(p.a && p.c && (p.ends || routed) && workspace, "%s: null pointer", fn);
+  EXQ_REQUIRE(((uintptr_t)p.a | (uintptr_t)workspace) % 16 == 0,
               "%s: A and workspace must be 16-byte aligned", fn);
   unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
   int* hdr = reinterpret_cast<int*>(ws);
-  TgEntry* tg = reinterpret_cast<TgEntry*>(ws + tg_off);
-  const bool bf = act_dtype == EXQ_DTYPE_BF16;
-  const bool tile = !general && (tier == 2 || tier == 0) &&
-                    tile_gemm_applies(tier, MODE_PLAIN, (int)N, 0, (int)K, (int)gs) &&
-                    tile_rowsum_floats(n_rows, K) * 4 <= 0x7fffffffLL;
-  int st = launch_tg_from_ends(ends, (int)n_experts, mask, tier,
-                               general ? kTokenGroupRows : (tile ? kTokenGroupI4 : kTokenGroup), hdr, tg,
-                               (int)tg_cap, s);
+  TgEntry* tg = reinterpret_cast<TgEntry*>(ws + L.tg);
+  const bool bf = p.act_dtype == EXQ_DTYPE_BF16;
+  // Few rows per expert, and shapes that the tiles do not take: the rows
+  // kernels, as in the fused layer.  Otherwise the tiles, INT4 as 64 x 256 up to
+  // 512 rows per expert.
+  const bool few = n_rows <= (p.tier == 2 ? kTokenGroupRows : kRowsBf16Max) * p.E;
+  const bool x32 = !routed || p.n_tokens * K * 2 <= 0x7fffffffLL;
+  const bool tile = !general && !few && x32 &&
+                    tile_gemm_applies(p.tier, MODE_PLAIN, (int)N, 0, (int)K, (int)gs) &&
+                    tile_rowsum_floats(rs_rows, K) * 4 <= 0x7fffffffLL;
+  const int shape = p.tier == 2 && tile_gemm_wide_applies(MODE_PLAIN, (int)N, 0) &&
+                            n_rows < 512 * p.E
+                        ? TILE_64x256
+                        : TILE_128x128;
+  const int group = !tile                    ? kTokenGroupRows
+                    : shape == TILE_128x128 ? kTokenGroupI4
+                                            : kTokenGroup;
+  int* sorted = reinterpret_cast<int*>(ws + L.sorted);
+  int st;
+  if (routed) {
+    RoutePlanParams rp{};
+    rp.ids = p.ids;
+    rp.ids_dtype = p.ids_dtype;
+    rp.T = (int)p.n_tokens;
+    rp.k = rp.kp = (int)p.top_k;
+    rp.E = rp.Ep = (int)p.E;
+    rp.n = (int)n_rows;
+    rp.all_tier = p.tier;
+    rp.mask = p.mask;
+    rp.hdr = hdr;
+    rp.ends = reinterpret_cast<int*>(ws + L.ends);
+    rp.sorted = sorted;
+    rp.tg = tg;
+    rp.tg_cap = (int)L.tg_cap;
+    rp.i4_group = rp.bf_group = rp.i8_group = group;
+    rp.blk_cnt = reinterpret_cast<int*>(ws + L.blk);
+    st = launch_route_plan(rp, s);
+  } else {
+    st = launch_tg_from_ends(p.ends, (int)p.E, p.mask, p.tier, group, hdr, tg, (int)L.tg_cap, s);
+  }
   if (st) return st;
   GemmArgs g{};
   g.hdr = hdr;
   g.tg = tg;
-  g.n_blocks = (int)(N / 32);
-  g.x = reinterpret_cast<const uint16_t*>(a_sorted);
+  g.x = reinterpret_cast<const uint16_t*>(p.a);
   g.x_stride = K;
+  g.row_slot = sorted;
+  g.gather = routed ? 1 : 0;
+  g.slot_div = routed ? (int)p.top_k : 1;
   g.K = (int)K;
-  g.w = bank;
+  g.w = p.bank;
   g.n_rows = (int)N;
   g.group_size = (int)gs;
-  g.out = c;
+  g.out = p.c;
   g.out_stride = N;
-  if (general) return launch_rows_gemm(MODE_PLAIN, bf, g, tg_cap, s);
-  if (tile && tier == 0) return launch_tile_gemm(0, MODE_PLAIN, bf, g, nullptr, 0, 0, tg_cap, s);
-  if (tile) {
-    float* rs = reinterpret_cast<float*>(ws + rs_off);
-    st = launch_group_rowsum(bf, g.x, K, n_rows, (int)K, (int)gs, rs, s);
-    if (st) return st;
-    return launch_tile_gemm(2, MODE_PLAIN, bf, g, rs, n_rows, 0, tg_cap, s);
-  }
-  return launch_gemm<MODE_PLAIN>(bf, g, tg_cap * g.n_blocks, s);
+  if (!tile)
+    return p.tier == 2 ? launch_rows_gemm(MODE_PLAIN, bf, g, L.tg_cap, s)
+                       : launch_rows_gemm_bf16(bf, g, L.tg_cap, s);
+  const int64_t xb = routed ? p.n_tokens * K * 2 : 0;
+  if (p.tier == 0) return launch_tile_gemm(0, MODE_PLAIN, bf, g, nullptr, 0, xb, L.tg_cap, s);
+  float* rs = reinterpret_cast<float*>(ws + L.rs);
+  st = launch_group_rowsum(bf, g.x, K, rs_rows, (int)K, (int)gs, rs, s);
+  if (st) return st;
+  return launch_tile_gemm(2, MODE_PLAIN, bf, g, rs, rs_rows, xb, L.tg_cap, s, shape);
 }
 
 }  // namespace
@@ -914,9 +983,13 @@ extern "C" int exq_set_stage_events(void* const* events, int n_events) {
 
 extern "C" size_t exq_moe_gemm_workspace_size(int64_t n_rows, int64_t n_experts, int64_t K) {
   const int64_t r = n_rows > 0 ? n_rows : 0;
-  return align_up(64, 256) + align_up((size_t)tg_capacity(r, n_experts, kTokenGroupRows) * sizeof(TgEntry),
-                                        256) +
-         align_up((size_t)tile_rowsum_floats(r, K > 0 ? K : 0) * 4, 256);
+  return sorted_layout(r, r, n_experts, K > 0 ? K : 0, false).total;
+}
+
+extern "C" size_t exq_moe_routed_gemm_workspace_size(int64_t n_tokens, int64_t top_k,
+                                                     int64_t n_experts, int64_t K) {
+  const int64_t t = n_tokens > 0 ? n_tokens : 0;
+  return sorted_layout(t * top_k, t, n_experts, K > 0 ? K : 0, true).total;
 }
 
 extern "C" int exq_moe_int4_fused_forward(const exq_moe_problem* problem, const void* hidden,
@@ -976,12 +1049,17 @@ extern "C" int exq_moe_int4_gemm(const void* a_sorted, int act_dtype, int64_t n_
                                  size_t workspace_bytes, exq_stream stream) {
   const char* fn = "exq_moe_int4_gemm";
   EXQ_REQUIRE(packed && scales, "%s: null weights", fn);
-  Bank b{};
-  b.i4 = packed;
-  b.i4_scales = scales;
-  return sorted_gemm_impl(a_sorted, act_dtype, n_rows, K, b, 2, n_experts, N, group_size,
-                          expert_ends, nullptr, c, workspace, workspace_bytes,
-                          as_stream(stream), fn);
+  SortedGemm p{};
+  p.a = a_sorted;
+  p.act_dtype = act_dtype;
+  p.n_rows = n_rows;
+  p.K = K; p.E = n_experts; p.N = N; p.gs = group_size;
+  p.bank.i4 = packed;
+  p.bank.i4_scales = scales;
+  p.tier = 2;
+  p.ends = expert_ends;
+  p.c = c;
+  return sorted_gemm_impl(p, workspace, workspace_bytes, as_stream(stream), fn);
 }
 
 extern "C" int exq_moe_grouped_gemm(const void* a_sorted, int act_dtype, int64_t n_rows,
@@ -991,9 +1069,48 @@ extern "C" int exq_moe_grouped_gemm(const void* a_sorted, int act_dtype, int64_t
                                     size_t workspace_bytes, exq_stream stream) {
   const char* fn = "exq_moe_grouped_gemm";
   EXQ_REQUIRE(weights, "%s: null weights", fn);
-  Bank b{};
-  b.bf16 = reinterpret_cast<const uint16_t*>(weights);
-  return sorted_gemm_impl(a_sorted, act_dtype, n_rows, K, b, 0, n_experts, N, 128,
-                          expert_ends, expert_mask, c, workspace, workspace_bytes,
-                          as_stream(stream), fn);
+  SortedGemm p{};
+  p.a = a_sorted;
+  p.act_dtype = act_dtype;
+  p.n_rows = n_rows;
+  p.K = K; p.E = n_experts; p.N = N; p.gs = 128;
+  p.bank.bf16 = reinterpret_cast<const uint16_t*>(weights);
+  p.tier = 0;
+  p.ends = expert_ends;
+  p.mask = expert_mask;
+  p.c = c;
+  return sorted_gemm_impl(p, workspace, workspace_bytes, as_stream(stream), fn);
+}
+
+extern "C" int exq_moe_routed_gemm(const void* hidden, int act_dtype, int64_t n_tokens, int64_t K,
+                                   const void* router_indices, int ids_dtype, int64_t top_k,
+                                   const uint8_t* packed, const uint16_t* scales,
+                                   const void* weights, int64_t n_experts, int64_t N,
+                                   int64_t group_size, const int32_t* expert_mask, void* c,
+                                   void* workspace, size_t workspace_bytes, exq_stream stream) {
+  const char* fn = "exq_moe_routed_gemm";
+  EXQ_REQUIRE((packed && scales) || (weights && !packed), "%s: null weights", fn);
+  EXQ_REQUIRE(is_index_dtype(ids_dtype), "%s: ids dtype must be i32 or i64", fn);
+  EXQ_REQUIRE(n_tokens >= 0 && top_k >= 1 && n_tokens <= INT32_MAX, "%s: bad sizes", fn);
+  EXQ_REQUIRE(n_tokens * top_k <= (1 << 24), "%s: %lld slots exceed 2^24", fn,
+              (long long)(n_tokens * top_k));
+  if (n_tokens == 0) return EXQ_SUCCESS;
+  EXQ_REQUIRE(router_indices, "%s: null pointer", fn);
+  SortedGemm p{};
+  p.a = hidden;
+  p.act_dtype = act_dtype;
+  p.n_rows = n_tokens * top_k;
+  p.K = K; p.E = n_experts; p.N = N;
+  p.gs = packed ? group_size : 128;
+  p.bank.i4 = packed;
+  p.bank.i4_scales = scales;
+  p.bank.bf16 = reinterpret_cast<const uint16_t*>(weights);
+  p.tier = packed ? 2 : 0;
+  p.mask = expert_mask;
+  p.ids = router_indices;
+  p.ids_dtype = ids_dtype;
+  p.n_tokens = n_tokens;
+  p.top_k = top_k;
+  p.c = c;
+  return sorted_gemm_impl(p, workspace, workspace_bytes, as_stream(stream), fn);
 }

@@ -200,15 +200,32 @@ __device__ __forceinline__ int tile_brow(int wn, int t) {
     return wn * NTW * 16 + t * 16;
 }
 
-// Activation row (GATEUP: token) of tile row m; rows past the group repeat
+// Whether the tile's rows are gathered tokens (GATEUP, and PLAIN on request)
+// or consecutive expert-sorted rows.
+template <int MODE>
+__device__ __forceinline__ bool tile_gather(const GemmArgs& a) {
+  return MODE == MODE_GATEUP || (MODE == MODE_PLAIN && a.gather);
+}
+
+// Activation row (gathered: token) of tile row m; rows past the group repeat
 // its last row (finite values whose outputs are never stored).
 template <int MODE>
 __device__ __forceinline__ int tile_xrow(const GemmArgs& a, const TgEntry& te, int m) {
   const int mm = m < te.cnt ? m : te.cnt - 1;
-  if constexpr (MODE == MODE_GATEUP)
+  if (tile_gather<MODE>(a))
     return a.row_slot[te.pos0 + mm] / a.slot_div;
   else
     return te.pos0 + mm;
+}
+
+// The activation rows as a buffer resource: all tokens when gathered, the
+// group's own rows otherwise.
+template <int MODE>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_xrsrc(const GemmArgs& a, const TgEntry& te,
+                                                            int64_t x_bytes) {
+  const bool g = tile_gather<MODE>(a);
+  return make_rsrc(g ? a.x : a.x + (int64_t)te.pos0 * a.x_stride,
+                   g ? x_bytes : (int64_t)te.cnt * a.x_stride * 2);
 }
 
 // Store a wave's finished sub-tile (rows wm*MT*16.., MFMA output layout) of a
@@ -320,7 +337,7 @@ __device__ __forceinline__ void tile_gemm_body(const GemmArgs& a, const TileArgs
   int nt;
   if (!tile_unit(a, a.hdr[ta.h_lo], a.hdr[ta.h_hi] - a.hdr[ta.h_lo], ta.n_tiles, bid, te, nt))
     return;  // INT4 groups [hdr[h_lo], hdr[h_hi])
-  const int cnt = te.cnt, pos0 = te.pos0;
+  const int pos0 = te.pos0;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: LDS DMA bases in SGPRs
@@ -341,10 +358,7 @@ __device__ __forceinline__ void tile_gemm_body(const GemmArgs& a, const TileArgs
       make_rsrc(a.w.i4 + ebase * rowbytes, (int64_t)a.n_rows * rowbytes);
   const __amdgpu_buffer_rsrc_t sr =
       make_rsrc(a.w.i4_scales + ebase * ngs, (int64_t)a.n_rows * ngs * 2);
-  const __amdgpu_buffer_rsrc_t xr =
-      MODE == MODE_GATEUP
-          ? make_rsrc(a.x, ta.x_bytes)
-          : make_rsrc(a.x + (int64_t)pos0 * a.x_stride, (int64_t)cnt * a.x_stride * 2);
+  const __amdgpu_buffer_rsrc_t xr = tile_xrsrc<MODE>(a, te, ta.x_bytes);
   const __amdgpu_buffer_rsrc_t rr = make_rsrc(ta.rs, (int64_t)ngs * ta.rs_rows * 4);
   const __amdgpu_buffer_rsrc_t wnull = make_rsrc(a.w.i4, 0);
   const __amdgpu_buffer_rsrc_t snull = make_rsrc(a.w.i4_scales, 0);
@@ -358,7 +372,7 @@ __device__ __forceinline__ void tile_gemm_body(const GemmArgs& a, const TileArgs
     const int m = (wave * QA + q) * 4 + (lane >> 4);
     const int c = (lane & 15) ^ a_swz(m & 15);
     const int xrow = x_row(m);
-    voffA[q] = (MODE == MODE_GATEUP ? xrow : xrow - pos0) * (int)a.x_stride * 2 + c * 16;
+    voffA[q] = (tile_gather<MODE>(a) ? xrow : xrow - pos0) * (int)a.x_stride * 2 + c * 16;
   }
 #pragma unroll
   for (int q = 0; q < QB; ++q) {  // LDS rows 16j..16j+15 per instruction, 4 columns each
@@ -671,7 +685,7 @@ __device__ __forceinline__ void tile_ps_body(const GemmArgs& a, const TileArgs& 
   int nt;
   if (!tile_unit(a, a.hdr[ta.h_lo], a.hdr[ta.h_hi] - a.hdr[ta.h_lo], ta.n_tiles, bid, te, nt))
     return;  // INT4 groups [hdr[h_lo], hdr[h_hi])
-  const int cnt = te.cnt, pos0 = te.pos0;
+  const int pos0 = te.pos0;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -691,10 +705,7 @@ __device__ __forceinline__ void tile_ps_body(const GemmArgs& a, const TileArgs& 
       make_rsrc(a.w.i4 + ebase * rowbytes, (int64_t)a.n_rows * rowbytes);
   const __amdgpu_buffer_rsrc_t sr =
       make_rsrc(a.w.i4_scales + ebase * ngs, (int64_t)a.n_rows * ngs * 2);
-  const __amdgpu_buffer_rsrc_t xr =
-      MODE == MODE_GATEUP
-          ? make_rsrc(a.x, ta.x_bytes)
-          : make_rsrc(a.x + (int64_t)pos0 * a.x_stride, (int64_t)cnt * a.x_stride * 2);
+  const __amdgpu_buffer_rsrc_t xr = tile_xrsrc<MODE>(a, te, ta.x_bytes);
   const __amdgpu_buffer_rsrc_t wnull = make_rsrc(a.w.i4, 0);
   const __amdgpu_buffer_rsrc_t snull = make_rsrc(a.w.i4_scales, 0);
   const __amdgpu_buffer_rsrc_t xnull = make_rsrc(a.x, 0);
@@ -708,7 +719,7 @@ __device__ __forceinline__ void tile_ps_body(const GemmArgs& a, const TileArgs& 
     const int m = (wave * QA + q) * 8 + (lane >> 3);
     const int c = (lane & 7) ^ psa_swz(m);
     const int xrow = x_row(m);
-    voffA[q] = (MODE == MODE_GATEUP ? xrow : xrow - pos0) * (int)a.x_stride * 2 + c * 16;
+    voffA[q] = (tile_gather<MODE>(a) ? xrow : xrow - pos0) * (int)a.x_stride * 2 + c * 16;
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -901,7 +912,7 @@ __device__ __forceinline__ void tile_i8_body(const GemmArgs& a, const TileArgs& 
   int nt;
   if (!tile_unit(a, a.hdr[ta.h_lo], a.hdr[ta.h_hi] - a.hdr[ta.h_lo], ta.n_tiles, bid, te, nt))
     return;  // INT8 groups [hdr[h_lo], hdr[h_hi])
-  const int cnt = te.cnt, pos0 = te.pos0;
+  const int pos0 = te.pos0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r32 = lane & 31, h = lane >> 5;
@@ -912,10 +923,7 @@ __device__ __forceinline__ void tile_i8_body(const GemmArgs& a, const TileArgs& 
   const int64_t ebase = (int64_t)widx * a.n_rows;
 
   const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.w.i8 + ebase * K, (int64_t)a.n_rows * K);
-  const __amdgpu_buffer_rsrc_t xr =
-      MODE == MODE_GATEUP
-          ? make_rsrc(a.x, ta.x_bytes)
-          : make_rsrc(a.x + (int64_t)pos0 * a.x_stride, (int64_t)cnt * a.x_stride * 2);
+  const __amdgpu_buffer_rsrc_t xr = tile_xrsrc<MODE>(a, te, ta.x_bytes);
   const __amdgpu_buffer_rsrc_t wnull = make_rsrc(a.w.i8, 0);
   const __amdgpu_buffer_rsrc_t xnull = make_rsrc(a.x, 0);
 
@@ -926,7 +934,7 @@ __device__ __forceinline__ void tile_i8_body(const GemmArgs& a, const TileArgs& 
   for (int q = 0; q < 4; ++q) {
     const int m = (wave * 4 + q) * 8 + (lane >> 3);
     const int xrow = tile_xrow<MODE>(a, te, m);
-    voffA[q] = (MODE == MODE_GATEUP ? xrow : xrow - pos0) * (int)a.x_stride * 2 +
+    voffA[q] = (tile_gather<MODE>(a) ? xrow : xrow - pos0) * (int)a.x_stride * 2 +
                ((lane & 7) ^ psa_swz(m)) * 16;
     const int rho = (wave * 4 + q) * 16 + (lane >> 2);
     voffB[q] = tile_wrow<MODE, TN>(a, nt, rho) * K + ((lane & 3) ^ psb_swz(rho)) * 16;
@@ -1025,7 +1033,7 @@ __device__ __forceinline__ void tile_gemm_bf16_body(const GemmArgs& a, const Til
   TgEntry te;
   int nt;
   if (!tile_unit(a, 0, a.hdr[2], ta.n_tiles, bid, te, nt)) return;  // BF16 groups
-  const int cnt = te.cnt, pos0 = te.pos0;
+  const int pos0 = te.pos0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, kq = lane >> 4;
@@ -1038,10 +1046,7 @@ __device__ __forceinline__ void tile_gemm_bf16_body(const GemmArgs& a, const Til
 
   const __amdgpu_buffer_rsrc_t wr =
       make_rsrc(a.w.bf16 + ebase * K, (int64_t)a.n_rows * rowbytes);
-  const __amdgpu_buffer_rsrc_t xr =
-      MODE == MODE_GATEUP
-          ? make_rsrc(a.x, ta.x_bytes)
-          : make_rsrc(a.x + (int64_t)pos0 * a.x_stride, (int64_t)cnt * a.x_stride * 2);
+  const __amdgpu_buffer_rsrc_t xr = tile_xrsrc<MODE>(a, te, ta.x_bytes);
   const __amdgpu_buffer_rsrc_t wnull = make_rsrc(a.w.bf16, 0);
   const __amdgpu_buffer_rsrc_t xnull = make_rsrc(a.x, 0);
 
@@ -1053,7 +1058,7 @@ __device__ __forceinline__ void tile_gemm_bf16_body(const GemmArgs& a, const Til
     const int r = (wave * 4 + q) * 8 + (lane >> 3);
     const int c = (lane & 7) ^ bf_swz(r & 15);
     const int xrow = tile_xrow<MODE>(a, te, r);
-    voffA[q] = (MODE == MODE_GATEUP ? xrow : xrow - pos0) * (int)a.x_stride * 2 + c * 16;
+    voffA[q] = (tile_gather<MODE>(a) ? xrow : xrow - pos0) * (int)a.x_stride * 2 + c * 16;
     voffB[q] = tile_wrow<MODE>(a, nt, r) * rowbytes + c * 16;
   }
   // Fragment of k-step s: column (2 kq + s) ^ f(r16) of the row.

@@ -235,6 +235,19 @@ __global__ void __launch_bounds__(RT) dispatch_kernel(const void* ids, int ids_d
       });
 }
 
+// The same sort as inverse positions only (exq_unsort_combine).
+__global__ void __launch_bounds__(RT) inverse_sort_kernel(const void* ids, int ids_dtype, int n,
+                                                          int E, int32_t* inv) {
+  __shared__ RouteLds s;
+  block_sort_any(
+      n, E + 1, s,
+      [&](int i) -> int {
+        const int64_t v = load_index(ids, ids_dtype, i);
+        return (v >= 0 && v < E) ? (int)v : E;
+      },
+      [](int c) { return c; }, []() {}, [&](int i, int, int pos) { inv[i] = pos; });
+}
+
 // ---- exq_build_ends_from_slots ---------------------------------------------
 __global__ void __launch_bounds__(RT) build_ends_kernel(const int32_t* sid, int em,
                                                         const int32_t* fr, int n_active, int E,
@@ -549,8 +562,8 @@ __device__ void plan_tail(const RoutePlanParams& p, RouteLds& s) {
   if (p.ends_out) {
     for (int e = threadIdx.x; e <= p.E; e += RT) p.ends_out[e] = s.start[e];
   }
-  const int c = b < nb ? s.cnt[b] : 0;
-  const int my_tier = (b < nb) ? (p.tier ? (int)p.tier[b] : 2) : -1;
+  const int c = b < nb && !(p.mask && p.mask[b] == 0) ? s.cnt[b] : 0;
+  const int my_tier = (b < nb) ? (p.tier ? (int)p.tier[b] : p.all_tier) : -1;
   // list class of the bucket's groups: 0 BF16, 1 INT8, 2 INT4 experts with at
   // least i4_big_rows rows, 3 the other INT4 experts
   const int my_cls =
@@ -807,6 +820,14 @@ int launch_route_plan(const RoutePlanParams& p, hipStream_t stream) {
   if (st) return st;
   hipLaunchKernelGGL(route_scatter_kernel, dim3((unsigned)nblk), dim3(RT), 0, stream, p);
   return check_launch("route_scatter_kernel");
+}
+
+bool inverse_sort_fits(int64_t n, int64_t nb) { return sort_fits(n, nb); }
+
+int launch_inverse_sort(const void* ids, int ids_dtype, int n, int E, int32_t* inv,
+                        hipStream_t stream) {
+  hipLaunchKernelGGL(inverse_sort_kernel, dim3(1), dim3(RT), 0, stream, ids, ids_dtype, n, E, inv);
+  return check_launch("inverse_sort_kernel");
 }
 
 int launch_tg_from_ends(const int32_t* ends, int E, const int32_t* expert_mask, int tier,

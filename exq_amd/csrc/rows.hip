@@ -186,7 +186,9 @@ __device__ __forceinline__ void rows_body(const GemmArgs& a, int n_tiles, unsign
   for (int q = 0; q < QA; ++q) {
     const int m = (wave * QA + q) * 4 + (lane >> 4);
     const int mm = m < cnt ? m : cnt - 1;  // rows past the group repeat its last row
-    const int64_t row = MODE == MODE_GATEUP ? a.row_slot[pos0 + mm] / a.slot_div : pos0 + mm;
+    const int64_t row = MODE == MODE_GATEUP || (MODE == MODE_PLAIN && a.gather)
+                            ? a.row_slot[pos0 + mm] / a.slot_div
+                            : pos0 + mm;
     cA[q] = ((lane & 15) ^ ra_swz(m & 15)) * 8;  // k of this lane's piece in the chunk
     pA[q] = a.x + row * a.x_stride + cA[q];
   }
@@ -400,6 +402,118 @@ __global__ void __launch_bounds__(RTH, 4) rows_kernel(GemmArgs a, int n_tiles) {
   rows_body<BF, MODE, SPG>(a, n_tiles, sA0, sA1, sB0, sB1);
 }
 
+// Unquantised weights: C = A x W^T with the same 32-row x 128-weight-row
+// work-groups, in chunks of 64 k (32 rows x 128 B and 128 rows x 128 B, whole
+// cache lines; 40 KiB of LDS for two stages, four work-groups per CU with 64 KiB
+// of weights in flight).  Lane (r, q) at k-step s holds k = 32 s + 8 q .. + 7 of
+// both operands, both LDS images swizzled by w_swz (free of bank conflicts);
+// the fp32 accumulators run over the whole contraction.
+//
+// Bound: HBM, the weights of the active experts read once.  OLMoE shape (K =
+// 2048, 2048 weight rows) at 96 tokens: 115 us on the 128 x 128 tiles (whose
+// activation rows are mostly padding there) -> 107 us.
+constexpr int WKC = 64;
+__device__ __forceinline__ int w_swz(int r) { return (r >> 1) & 7; }
+
+template <bool BF>
+__global__ void __launch_bounds__(RTH, 4) rows_bf16_kernel(GemmArgs a, int n_tiles) {
+  __shared__ __attribute__((aligned(1024))) unsigned char sA0[MT * 16 * WKC * 2];
+  __shared__ __attribute__((aligned(1024))) unsigned char sA1[MT * 16 * WKC * 2];
+  __shared__ __attribute__((aligned(1024))) unsigned char sB0[TN * WKC * 2];
+  __shared__ __attribute__((aligned(1024))) unsigned char sB1[TN * WKC * 2];
+  static_assert(MT == 2, "one activation copy per wave and chunk");
+  constexpr int QB = TN / 32;  // weight copies per wave and chunk (8 rows each)
+  TgEntry te;
+  int nt;
+  if (!rows_unit(a, 0, a.hdr[2], n_tiles, blockIdx.x, te, nt)) return;  // BF16 groups
+  nt = uni_i(nt);
+  const int cnt = uni_i(te.cnt), pos0 = uni_i(te.pos0);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, kq = lane >> 4;
+  const int K = a.K, nch = K / WKC;  // an even number of chunks: K % 128 == 0
+  const int c0 = nt * TN;
+  const int left = a.n_rows - c0;
+  const int have = left < TN ? left : TN;
+  const int e = uni_i(te.e);
+  const int64_t row0 = (int64_t)(a.w.index ? uni_i(a.w.index[e]) : e) * a.n_rows + c0;
+  const __amdgpu_buffer_rsrc_t wr = rsrc32(a.w.bf16 + row0 * K, have * K * 2);
+
+  // copies: 8 rows x 8 columns of 16 bytes per instruction
+  const int m = wave * 8 + (lane >> 3);
+  const int mm = m < cnt ? m : cnt - 1;  // rows past the group repeat its last row
+  const int64_t xrow = a.gather ? a.row_slot[pos0 + mm] / a.slot_div : pos0 + mm;
+  const uint16_t* pA = a.x + xrow * a.x_stride + ((lane & 7) ^ w_swz(m & 15)) * 8;
+  int vB[QB];
+#pragma unroll
+  for (int q = 0; q < QB; ++q) {
+    const int rho = (wave * QB + q) * 8 + (lane >> 3);
+    const int l = rho < have ? rho : have - 1;  // rows past the end repeat the last one
+    vB[q] = l * K * 2 + ((lane & 7) ^ w_swz(rho & 15)) * 16;
+  }
+  auto copy = [&](unsigned char* A, unsigned char* B, int ch) {
+    if (ch >= nch) return;
+#pragma unroll
+    for (int q = 0; q < QB; ++q)
+      bdma16(wr, B + (wave * QB + q) * 1024, vB[q], uni_i(ch * WKC * 2));
+    gdma16(pA + (int64_t)ch * WKC, A + wave * 1024);
+  };
+  f32x4_t acc[MT][NTW];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int t = 0; t < NTW; ++t) acc[mt][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int swz = w_swz(r16);
+  auto chunk = [&](const unsigned char* A, const unsigned char* B) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      uint4 af[MT], bf[NTW];
+      const int col = ((4 * s + kq) ^ swz) * 16;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        af[mt] = *reinterpret_cast<const uint4*>(A + (mt * 16 + r16) * 128 + col);
+#pragma unroll
+      for (int t = 0; t < NTW; ++t)
+        bf[t] = *reinterpret_cast<const uint4*>(B + ((wave * NTW + t) * 16 + r16) * 128 + col);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int t = 0; t < NTW; ++t) acc[mt][t] = dmfma<BF>(af[mt], bf[t], acc[mt][t]);
+    }
+  };
+  auto barrier = [&]() {  // as in rows_body
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  copy(sA0, sB0, 0);
+  for (int ch = 0; ch < nch; ch += 2) {
+    barrier();
+    copy(sA1, sB1, ch + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    chunk(sA0, sB0);
+    barrier();
+    copy(sA0, sB0, ch + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    chunk(sA1, sB1);
+  }
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int mr = mt * 16 + kq * 4 + i;
+      if (mr >= cnt) continue;
+      uint16_t* c = reinterpret_cast<uint16_t*>(a.out) + (int64_t)(pos0 + mr) * a.out_stride + c0;
+#pragma unroll
+      for (int t = 0; t < NTW; ++t) {
+        const int col = (wave * NTW + t) * 16 + r16;
+        if (col < have) c[col] = (uint16_t)to_act_bits<BF>(acc[mt][t][i]);
+      }
+    }
+  }
+}
+
 template <int MODE, int SPG>
 int launch_spg(bool bf, const GemmArgs& a, int64_t grid, int n_tiles, hipStream_t s) {
   const dim3 g((unsigned)grid), b(RTH);
@@ -437,6 +551,21 @@ int launch_rows_gemm(int mode, bool bf, const GemmArgs& a, int64_t tg_cap, hipSt
   if (mode == MODE_GATEUP) return launch_mode<MODE_GATEUP>(bf, a, tg_cap, s);
   if (mode == MODE_DOWN) return launch_mode<MODE_DOWN>(bf, a, tg_cap, s);
   return launch_mode<MODE_PLAIN>(bf, a, tg_cap, s);
+}
+
+int launch_rows_gemm_bf16(bool bf, const GemmArgs& a, int64_t tg_cap, hipStream_t s) {
+  if (a.K > (1 << 22))  // 32-bit offsets inside a tile's weight rows
+    return set_error(EXQ_ERROR_UNSUPPORTED, "rows_gemm: contraction of %d too long", a.K);
+  const int n_tiles = (int)cdiv(a.n_rows, TN);
+  const int64_t grid = 8 * cdiv(tg_cap, 8) * n_tiles;
+  if (grid <= 0) return EXQ_SUCCESS;
+  if (grid > INT32_MAX) return set_error(EXQ_ERROR_UNSUPPORTED, "rows_gemm: problem too large");
+  const dim3 g((unsigned)grid), b(RTH);
+  if (bf)
+    hipLaunchKernelGGL(rows_bf16_kernel<true>, g, b, 0, s, a, n_tiles);
+  else
+    hipLaunchKernelGGL(rows_bf16_kernel<false>, g, b, 0, s, a, n_tiles);
+  return check_launch("rows_bf16_kernel");
 }
 
 }  // namespace exq

@@ -9,7 +9,8 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from .exq_dispatch import combine, dispatch, gather_hidden
+from .exq_dispatch import dispatch, gather_hidden
+from .moe_int4_kernel import routed_gemm
 
 
 def sort_tokens_by_expert(router_indices: torch.Tensor, hidden_states: torch.Tensor,
@@ -56,23 +57,12 @@ def moe_grouped_gemm(hidden_states: torch.Tensor, expert_weights: torch.Tensor,
         raise ValueError("expert_weights must have the activation dtype")
     top_k = router_indices.shape[1]
     n_active = n_tok * top_k
-    ids = router_indices.reshape(-1).contiguous()
-    sort_order = torch.empty(n_active, dtype=torch.int64, device=dev)
-    sorted_ids = torch.empty(n_active, dtype=torch.int64, device=dev)
-    ends = torch.empty(n_experts + 1, dtype=torch.int32, device=dev)
-    dispatch(ids, sort_order, sorted_ids, ends, n_experts)
-    a = torch.empty(n_active, K, dtype=hidden_states.dtype, device=dev)
-    gather_hidden(hidden_states.contiguous(), sort_order, a, top_k)
     out = torch.zeros(n_active, N, dtype=hidden_states.dtype, device=dev)
-    L = _lib.lib()
-    ws = _lib.workspace(dev, L.exq_moe_gemm_workspace_size(n_active, n_experts, K))
     mask = None
     if expert_mask is not None:
         mask = expert_mask.to(torch.int32).contiguous()
-    _lib.check(L.exq_moe_grouped_gemm(
-        a.data_ptr(), _lib.dtype_code(a.dtype), n_active, K, expert_weights.data_ptr(),
-        n_experts, N, ends.data_ptr(), _lib.ptr(mask), out.data_ptr(), ws.data_ptr(),
-        ws.numel(), _lib.stream_handle(dev)), "moe_grouped_gemm")
+    routed_gemm(hidden_states, router_indices, n_experts, N, 128, out, weights=expert_weights,
+                mask=mask, what="moe_grouped_gemm")
     return out
 
 
@@ -94,12 +84,16 @@ def unsort_output(sorted_output: torch.Tensor, router_indices: torch.Tensor,
     n = T * k
     if sorted_output.dim() != 2 or sorted_output.shape[0] != n:
         raise ValueError(f"sorted_output must be [{n}, N]")
+    if router_weights.shape != router_indices.shape:
+        raise ValueError("router_weights must be [T, k] like router_indices")
     E = 1023 if n_experts is None else int(n_experts)
-    ids = router_indices.reshape(-1).contiguous()
-    sort_order = torch.empty(n, dtype=torch.int64, device=dev)
-    sorted_ids = torch.empty(n, dtype=torch.int64, device=dev)
-    ends = torch.empty(E + 1, dtype=torch.int32, device=dev)
-    dispatch(ids, sort_order, sorted_ids, ends, E)
-    result = torch.empty(T, sorted_output.shape[1], dtype=sorted_output.dtype, device=dev)
-    combine(sorted_output.contiguous(), sort_order, router_weights.contiguous(), result)
+    N = sorted_output.shape[1]
+    result = torch.empty(T, N, dtype=sorted_output.dtype, device=dev)
+    L = _lib.lib()
+    ws = _lib.workspace(dev, L.exq_unsort_combine_workspace_size(T, k, E))
+    _lib.check(L.exq_unsort_combine(
+        sorted_output.data_ptr(), _lib.dtype_code(sorted_output.dtype),
+        router_indices.data_ptr(), _lib.dtype_code(router_indices.dtype),
+        router_weights.data_ptr(), _lib.dtype_code(router_weights.dtype), T, k, E, N,
+        result.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_handle(dev)), "unsort_output")
     return result

@@ -129,21 +129,56 @@ def moe_int4_forward(hidden_states: torch.Tensor, expert_packed: torch.Tensor,
     gs = _effective_group(K, expert_scales)
     top_k = router_indices.shape[1]
     n_active = n_tok * top_k
+    out = torch.empty(n_active, N, dtype=hidden_states.dtype, device=dev)
+    routed_gemm(hidden_states, router_indices, n_experts, N, gs, out, packed=expert_packed,
+                scales=expert_scales, what="moe_int4_forward")
+    return out
+
+
+# Slots that one routed GEMM call takes (exq_moe_routed_gemm).
+_MAX_ROUTED_SLOTS = 1 << 24
+
+
+def routed_gemm(hidden: torch.Tensor, router_indices: torch.Tensor, n_experts: int, N: int,
+                group_size: int, out: torch.Tensor, *, packed: torch.Tensor | None = None,
+                scales: torch.Tensor | None = None, weights: torch.Tensor | None = None,
+                mask: torch.Tensor | None = None, what: str = "routed_gemm") -> None:
+    """``out[r] = hidden[slot(r) // k] @ W[e].T`` over the stable sort of the
+    routed slots, INT4 (packed, scales) or unquantised (weights)."""
+    n_tok, K = hidden.shape
+    top_k = router_indices.shape[1]
+    n = n_tok * top_k
+    if router_indices.numel() != n:
+        raise ValueError("sort_order / sorted_expert_ids must have n = T*k entries")
+    L = _lib.lib()
+    if n <= _MAX_ROUTED_SLOTS:
+        ids = router_indices.contiguous()
+        dev = _lib.require_gpu(hidden, ids)
+        ws = _lib.workspace(dev, L.exq_moe_routed_gemm_workspace_size(n_tok, top_k, n_experts, K))
+        _lib.check(L.exq_moe_routed_gemm(
+            hidden.data_ptr(), _lib.dtype_code(hidden.dtype), n_tok, K, ids.data_ptr(),
+            _lib.dtype_code(ids.dtype), top_k, _lib.ptr(packed), _lib.ptr(scales),
+            _lib.ptr(weights), n_experts, N, group_size, _lib.ptr(mask), out.data_ptr(),
+            ws.data_ptr(), ws.numel(), _lib.stream_handle(dev)), what)
+        return
+    dev = hidden.device
     ids = router_indices.reshape(-1).contiguous()
-    sort_order = torch.empty(n_active, dtype=torch.int64, device=dev)
-    sorted_ids = torch.empty(n_active, dtype=torch.int64, device=dev)
+    sort_order = torch.empty(n, dtype=torch.int64, device=dev)
+    sorted_ids = torch.empty(n, dtype=torch.int64, device=dev)
     ends = torch.empty(n_experts + 1, dtype=torch.int32, device=dev)
     dispatch(ids, sort_order, sorted_ids, ends, n_experts)
-    a = torch.empty(n_active, K, dtype=hidden_states.dtype, device=dev)
-    gather_hidden(hidden_states, sort_order, a, top_k)
-    out = torch.empty(n_active, N, dtype=hidden_states.dtype, device=dev)
-    L = _lib.lib()
-    ws = _lib.workspace(dev, L.exq_moe_gemm_workspace_size(n_active, n_experts, K))
-    _lib.check(L.exq_moe_int4_gemm(
-        a.data_ptr(), _lib.dtype_code(a.dtype), n_active, K, expert_packed.data_ptr(),
-        expert_scales.data_ptr(), n_experts, N, gs, ends.data_ptr(), out.data_ptr(),
-        ws.data_ptr(), ws.numel(), _lib.stream_handle(dev)), "moe_int4_forward")
-    return out
+    a = torch.empty(n, K, dtype=hidden.dtype, device=dev)
+    gather_hidden(hidden, sort_order, a, top_k)
+    ws = _lib.workspace(dev, L.exq_moe_gemm_workspace_size(n, n_experts, K))
+    code, st = _lib.dtype_code(a.dtype), _lib.stream_handle(dev)
+    if packed is not None:
+        _lib.check(L.exq_moe_int4_gemm(
+            a.data_ptr(), code, n, K, packed.data_ptr(), scales.data_ptr(), n_experts, N,
+            group_size, ends.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), st), what)
+    else:
+        _lib.check(L.exq_moe_grouped_gemm(
+            a.data_ptr(), code, n, K, weights.data_ptr(), n_experts, N, ends.data_ptr(),
+            _lib.ptr(mask), out.data_ptr(), ws.data_ptr(), ws.numel(), st), what)
 
 
 def moe_int4_full_forward(hidden_states: torch.Tensor, w13_packed: torch.Tensor,

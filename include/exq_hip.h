@@ -156,6 +156,20 @@ int exq_combine(const void* down_out, int dtype, const int64_t* sort_order, int6
                 void* workspace, size_t workspace_bytes, exq_stream stream);
 
 /*
+ * result[t, :] = sum_j w[t, j] * sorted_rows[pos(t*k + j), :], pos the place of
+ * slot t*k + j in the stable sort of router_indices (exq_dispatch's order), fp32
+ * accumulation in the fixed order j = 0..k-1.  The sort and the combine in one
+ * call; replaces unsort_output (exq/kernels/moe_grouped_gemm.py:234-260).
+ * dtype, weights: f32 | f16 | bf16; ids i32 | i64; n_experts < 4096.
+ */
+size_t exq_unsort_combine_workspace_size(int64_t n_tokens, int64_t top_k, int64_t n_experts);
+int exq_unsort_combine(const void* sorted_rows, int dtype, const void* router_indices,
+                       int ids_dtype, const void* router_weights, int weights_dtype,
+                       int64_t n_tokens, int64_t top_k, int64_t n_experts, int64_t hidden_size,
+                       void* result, void* workspace, size_t workspace_bytes,
+                       exq_stream stream);
+
+/*
  * out[m, j] = silu(x[m, j]) * x[m, I + j] computed in fp32.  Replaces
  * sgl_kernel.silu_and_mul (call sites sglang_backend.py:137-140,
  * moe_int4_kernel.py:398-400).  dtype: f32 | f16 | bf16.
@@ -174,10 +188,10 @@ int exq_silu_and_mul(const void* input, int dtype, int64_t rows, int64_t inter,
  * A and C: f16 | bf16 (same dtype).  K % 32 == 0 and a group size that is a
  * multiple of 32 dividing K (the reference's minimum group is 32,
  * moe_int4_kernel.py:286-290); any N >= 1 (the reference masks the N tail).
- * K, group_size multiples of 128 with N % 32 == 0 take the tiled / grouped
- * kernels, other shapes the rows kernel.  exq_moe_gemm_workspace_size
- * covers the token-group list and, for INT4 weights with N % 128 == 0 (the
- * tiled kernel), the per-row group sums of A (n_rows * K / 128 floats).
+ * Few rows per expert, and shapes outside the tiled kernels (K % 128, N % 128,
+ * group sizes other than 128), take the rows kernels.  exq_moe_gemm_workspace_size
+ * covers the token-group list and, for the tiled INT4 kernels, the per-row group
+ * sums of A (n_rows * K / 128 floats).
  */
 size_t exq_moe_gemm_workspace_size(int64_t n_rows, int64_t n_experts, int64_t K);
 int exq_moe_int4_gemm(const void* a_sorted, int act_dtype, int64_t n_rows, int64_t K,
@@ -195,6 +209,25 @@ int exq_moe_grouped_gemm(const void* a_sorted, int act_dtype, int64_t n_rows, in
                          const void* weights, int64_t n_experts, int64_t N,
                          const int32_t* expert_ends, const int32_t* expert_mask,
                          void* c, void* workspace, size_t workspace_bytes, exq_stream stream);
+
+/*
+ * Both GEMMs straight from the routing: C[r, :] = hidden[t, :] @ W[e]^T for the
+ * rows r of the stable sort of router_indices [n_tokens, top_k] (slot t*k + j,
+ * expert e), rows of ids outside [0, n_experts) and of experts with a zero
+ * expert_mask entry left unwritten.  The rows are gathered by the GEMM.  INT4
+ * weights (packed, scales) or unquantised ones (weights, with packed and scales
+ * null), shapes as above; n_tokens * top_k <= 2^24.  Replaces the launch
+ * sequences of moe_int4_forward and moe_grouped_gemm
+ * (exq/kernels/moe_int4_kernel.py:245-327, moe_grouped_gemm.py:173-227).
+ */
+size_t exq_moe_routed_gemm_workspace_size(int64_t n_tokens, int64_t top_k, int64_t n_experts,
+                                          int64_t K);
+int exq_moe_routed_gemm(const void* hidden, int act_dtype, int64_t n_tokens, int64_t K,
+                        const void* router_indices, int ids_dtype, int64_t top_k,
+                        const uint8_t* packed, const uint16_t* scales, const void* weights,
+                        int64_t n_experts, int64_t N, int64_t group_size,
+                        const int32_t* expert_mask, void* c, void* workspace,
+                        size_t workspace_bytes, exq_stream stream);
 
 /* ---- weight quantisation -------------------------------------------------- */
 

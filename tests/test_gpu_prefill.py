@@ -347,3 +347,60 @@ def test_prefill_routing_plan_sizes(T, device):
                             w[rows])
     assert_close_rel(out[torch.from_numpy(rows).to(device)], ref, TOL,
                      f"prefill routing plan T={T} (64 rows)")
+
+
+@pytest.mark.parametrize("T,k,E,K,N", [
+    (9, 2, 8, 128, 160),      # few rows per expert: rows kernels, N not a multiple of their tile
+    (70, 4, 9, 384, 256),     # 31 rows per expert on average
+    (80, 4, 9, 384, 256),     # 35: 64 x 256 INT4 tiles, 128 x 128 unquantised ones
+    (300, 2, 6, 256, 384),    # N % 256 != 0: 128 x 128
+    (300, 2, 6, 256, 96),     # N % 128 != 0: rows kernels at any batch
+    (1200, 1, 2, 128, 256),   # 600 rows per expert: 128 x 128
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_routed_gemms(T, k, E, K, N, dtype, device):
+    """moe_int4_forward and moe_grouped_gemm gather their rows from the routing:
+    every kernel that the row count per expert selects, ragged groups, dropped
+    ids (rows past the routed ones: unwritten / zero) and a masked expert."""
+    from exq_amd.kernels import moe_grouped_gemm, moe_int4_forward, pack_experts_int4
+    banner(f"routed gemms T={T} k={k} E={E} K={K} N={N} {dtype}")
+    rng = np.random.default_rng(T + N)
+    ids = np.minimum(rng.geometric(0.25, (T, k)) - 1, E - 1).astype(np.int64)
+    ids[rng.random((T, k)) < 0.05] = -1
+    x = torch.from_numpy(rng.standard_normal((T, K)).astype(np.float32)).to(dtype).to(device)
+    w = torch.from_numpy((rng.standard_normal((E, N, K)) * 0.05).astype(np.float32)).to(dtype)
+    flat = ids.reshape(-1)
+    order = np.argsort(np.where(flat < 0, E, flat), kind="stable")
+    n = int((flat >= 0).sum())
+    ends = np.searchsorted(np.sort(np.where(flat < 0, E, flat)), np.arange(E + 1))
+    rows = x.float().cpu().numpy()[order // k]
+    tid = torch.from_numpy(ids).to(device)
+    p, s = pack_experts_int4(w.to(torch.float16).to(device), 128)
+    out = moe_int4_forward(x, p, s, tid, E)
+    ref = moe.grouped_gemm_sorted(rows[:n], quant.dequant_int4(p.cpu().numpy(), s.cpu().numpy()),
+                                  ends)
+    assert_close_rel(out[:n], ref[:n], TOL, f"routed int4 T={T} K={K} N={N} {dtype}")
+    mask = torch.ones(E, dtype=torch.int32)
+    mask[0] = 0
+    out = moe_grouped_gemm(x, w.to(device), tid, E, expert_mask=mask.to(device))
+    ref = moe.grouped_gemm_sorted(rows[:n], w.float().numpy(), ends)
+    ref[:ends[1]] = 0
+    assert_close_rel(out[:n], ref[:n], TOL, f"routed gemm T={T} K={K} N={N} {dtype}")
+    assert not out[n:].any() and not out[:ends[1]].any()
+
+
+@pytest.mark.parametrize("T,k,E", [(1, 1, 1), (40, 8, 64), (700, 4, 100), (1200, 4, 1023)])
+def test_unsort_output_routes(T, k, E, device):
+    """unsort_output on the one-work-group sort and on the multi-block one, with
+    out-of-range ids (they sort last and still count)."""
+    from exq_amd.kernels import unsort_output
+    banner(f"unsort_output T={T} k={k} E={E}")
+    rng = np.random.default_rng(T + E)
+    ids = rng.integers(-1, E + 1, (T, k))
+    y = torch.from_numpy(rng.standard_normal((T * k, 72)).astype(np.float32))
+    w = torch.from_numpy(rng.random((T, k)).astype(np.float32))
+    flat = ids.reshape(-1)
+    order = np.argsort(np.where((flat < 0) | (flat >= E), E, flat), kind="stable")
+    got = unsort_output(y.to(device), torch.from_numpy(ids).to(device), w.to(device), E)
+    ref = moe.combine(y.numpy(), order, w.numpy())
+    assert np.allclose(got.cpu().numpy(), ref, rtol=4e-6, atol=4e-6)  # fp32 sums of k products
