@@ -326,7 +326,6 @@ __device__ __forceinline__ void rows_body(const GemmArgs& a, int n_tiles, unsign
         const int st = ch * 4 + s;
         if ((st + 1) % spg == 0) flush(st / spg);
       }
-      __builtin_amdgcn_sched_barrier(0);  // one step's fragments live at a time
     }
   };
 
