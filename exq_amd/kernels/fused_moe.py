@@ -19,40 +19,52 @@ from .moe_int4_kernel import _effective_group, pack_experts_int4
 _EPS = torch.finfo(torch.float32).eps
 
 
-def _problem(hidden: torch.Tensor, topk_ids: torch.Tensor, topk_weights: torch.Tensor,
-             n_experts: int, inter: int, group_size: int, n_shared: int = 0) -> _lib.MoeProblem:
-    T, H = hidden.shape
-    p = _lib.MoeProblem()
-    p.n_tokens = T
-    p.hidden_size = H
-    p.inter_size = inter
-    p.n_experts = n_experts
-    p.top_k = topk_ids.shape[1]
-    p.n_shared = n_shared
-    p.group_size = group_size
-    p.act_dtype = _lib.dtype_code(hidden.dtype)
-    p.ids_dtype = _lib.dtype_code(topk_ids.dtype)
-    p.weights_dtype = _lib.dtype_code(topk_weights.dtype)
-    return p
+_ACT_DTYPES = (torch.float16, torch.bfloat16)
+_ID_DTYPES = (torch.int32, torch.int64)
+_WEIGHT_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
 
 def _check_routing(hidden, topk_weights, topk_ids):
     if hidden.dim() != 2:
         raise ValueError("hidden_states must be [T, H]")
-    if (topk_ids.dim() != 2 or topk_ids.shape != topk_weights.shape
-            or topk_ids.shape[0] != hidden.shape[0]):
+    shape = topk_ids.shape
+    if len(shape) != 2 or shape != topk_weights.shape or shape[0] != hidden.shape[0]:
         raise ValueError("topk_ids / topk_weights must both be [T, k]")
-    if hidden.dtype not in (torch.float16, torch.bfloat16):
+    if hidden.dtype not in _ACT_DTYPES:
         raise ValueError("hidden_states must be float16 or bfloat16")
-    if topk_ids.dtype not in (torch.int32, torch.int64):
+    if topk_ids.dtype not in _ID_DTYPES:
         raise ValueError("topk_ids must be int32 or int64")
-    if topk_weights.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+    if topk_weights.dtype not in _WEIGHT_DTYPES:
         raise ValueError("topk_weights must be float32, float16 or bfloat16")
+
+
+def _call(entry, hidden, topk_ids, topk_weights, n_experts, inter, n_shared, group_size,
+          weight_args, dev, out, sort_order_out, expert_ends_out, workspace, what):
+    """One fused-layer call: problem, workspace, launch."""
+    T, H = hidden.shape
+    k = topk_ids.shape[1]
+    if out is None:
+        out = torch.empty(T, H, dtype=hidden.dtype, device=dev)
+    code = _lib._TORCH_TO_CODE
+    st = _lib.stream_handle(dev)
+    ws = workspace
+    if ws is None:
+        ws = _lib.workspace(dev, _lib.moe_workspace_size(T, H, inter, n_experts, k, n_shared,
+                                                         group_size), "fused", st)
+    _lib.check(entry(
+        _lib.MoeProblem(T, H, inter, n_experts, k, n_shared, group_size, code[hidden.dtype],
+                        code[topk_ids.dtype], code[topk_weights.dtype]),
+        hidden.data_ptr(), topk_ids.data_ptr(), topk_weights.data_ptr(), *weight_args,
+        out.data_ptr(), _lib.ptr(sort_order_out), _lib.ptr(expert_ends_out), ws.data_ptr(),
+        ws.numel(), st), what)
+    return out
 
 
 def _check_outputs(hidden, topk_ids, n_experts, out, sort_order_out, expert_ends_out):
     """Caller-supplied output buffers are written through raw pointers by the
     kernels, so their sizes and dtypes are checked here, before any launch."""
+    if out is None and sort_order_out is None and expert_ends_out is None:
+        return
     T, H = hidden.shape
     if out is not None and (tuple(out.shape) != (T, H) or out.dtype != hidden.dtype):
         raise ValueError(f"out must be [{T}, {H}] with dtype {hidden.dtype}")
@@ -90,12 +102,12 @@ def fused_experts(hidden_states: torch.Tensor, w13_packed: torch.Tensor,
     if activation != "silu":
         raise ValueError(f"unsupported activation {activation!r} (only 'silu')")
     _check_routing(hidden_states, topk_weights, topk_ids)
-    T, H = hidden_states.shape
+    H = hidden_states.shape[1]
     if w13_packed.dim() != 3 or w2_packed.dim() != 3:
         raise ValueError("packed weights must be [E, N, K/2]")
     E, two_i, h2 = w13_packed.shape
     I = two_i // 2
-    if h2 * 2 != H or tuple(w2_packed.shape) != (E, H, I // 2):
+    if h2 * 2 != H or w2_packed.shape != (E, H, I // 2):
         raise ValueError("packed weight shapes do not match hidden / intermediate sizes")
     if w13_packed.dtype != torch.uint8 or w2_packed.dtype != torch.uint8:
         raise ValueError("packed weights must be uint8")
@@ -105,34 +117,21 @@ def fused_experts(hidden_states: torch.Tensor, w13_packed: torch.Tensor,
     gs = _effective_group(H, w13_scales)
     if _effective_group(I, w2_scales) != gs:
         raise ValueError("w13 and w2 must use the same group size")
-    if (tuple(w13_scales.shape) != (E, two_i, H // gs)
-            or tuple(w2_scales.shape) != (E, H, I // gs)):
+    if w13_scales.shape != (E, two_i, H // gs) or w2_scales.shape != (E, H, I // gs):
         raise ValueError("scale shapes do not match the packed weights")
     dev = _lib.require_gpu(hidden_states, w13_packed, w13_scales, w2_packed, w2_scales,
                            topk_weights, topk_ids, out, sort_order_out, expert_ends_out)
-    if out is None:
-        out = torch.empty(T, H, dtype=hidden_states.dtype, device=dev)
-    p = _problem(hidden_states, topk_ids, topk_weights, E, I, gs)
-    L = _lib.lib()
-    need = L.exq_moe_workspace_size(p)
-    ws = workspace if workspace is not None else _lib.workspace(dev, need, "fused")
-    _lib.check(L.exq_moe_int4_fused_forward(
-        p, hidden_states.data_ptr(), topk_ids.data_ptr(), topk_weights.data_ptr(),
-        w13_packed.data_ptr(), w13_scales.data_ptr(), w2_packed.data_ptr(),
-        w2_scales.data_ptr(), out.data_ptr(), _lib.ptr(sort_order_out),
-        _lib.ptr(expert_ends_out), ws.data_ptr(), ws.numel(), _lib.stream_handle(dev)),
-        "fused_experts")
-    return out
+    return _call(_lib.lib().exq_moe_int4_fused_forward, hidden_states, topk_ids, topk_weights, E,
+                 I, 0, gs, (w13_packed.data_ptr(), w13_scales.data_ptr(), w2_packed.data_ptr(),
+                            w2_scales.data_ptr()),
+                 dev, out, sort_order_out, expert_ends_out, workspace, "fused_experts")
 
 
 def moe_workspace_bytes(n_tokens: int, hidden: int, inter: int, n_experts: int, top_k: int,
                         n_shared: int = 0, group_size: int = 128) -> int:
     """Workspace bytes the fused entry points need for this problem size."""
-    p = _lib.MoeProblem(n_tokens=n_tokens, hidden_size=hidden, inter_size=inter,
-                        n_experts=n_experts, top_k=top_k, n_shared=n_shared,
-                        group_size=group_size, act_dtype=_lib.BF16, ids_dtype=_lib.I32,
-                        weights_dtype=_lib.F32)
-    return int(_lib.lib().exq_moe_workspace_size(p))
+    return _lib.moe_workspace_size(n_tokens, hidden, inter, n_experts, top_k, n_shared,
+                                   group_size)
 
 
 def quantize_int8_rows(w: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
@@ -254,13 +253,10 @@ class MixedExpertBank:
         return bank
 
     def c_bank(self) -> _lib.ExpertBank:
-        b = _lib.ExpertBank()
-        for name in ("tier", "index", "bf16_w13", "bf16_w2", "int8_w13", "int8_w13_scales",
-                     "int8_w2", "int8_w2_scales", "int4_w13", "int4_w13_scales", "int4_w2",
-                     "int4_w2_scales"):
-            t = getattr(self, name)
-            setattr(b, name, None if t is None else t.data_ptr())
-        return b
+        return _lib.ExpertBank(*map(_lib.ptr, (
+            self.tier, self.index, self.bf16_w13, self.bf16_w2, self.int8_w13,
+            self.int8_w13_scales, self.int8_w2, self.int8_w2_scales, self.int4_w13,
+            self.int4_w13_scales, self.int4_w2, self.int4_w2_scales)))
 
     def tensors(self) -> list[torch.Tensor]:
         return [t for t in (self.tier, self.index, self.bf16_w13, self.bf16_w2, self.int8_w13,
@@ -287,8 +283,7 @@ def fused_experts_mixed(hidden_states: torch.Tensor, bank: MixedExpertBank,
                         workspace: torch.Tensor | None = None) -> torch.Tensor:
     """Mixed BF16/INT8/INT4 MoE layer (plus shared experts) in one launch sequence."""
     _check_routing(hidden_states, topk_weights, topk_ids)
-    T, H = hidden_states.shape
-    if H != bank.hidden_size:
+    if hidden_states.shape[1] != bank.hidden_size:
         raise ValueError("hidden size does not match the bank")
     if bank.bf16_w13 is not None and bank.bf16_w13.dtype != hidden_states.dtype:
         raise ValueError("BF16-tier weights must have the activation dtype")
@@ -296,16 +291,7 @@ def fused_experts_mixed(hidden_states: torch.Tensor, bank: MixedExpertBank,
                    expert_ends_out)
     dev = _lib.require_gpu(hidden_states, topk_weights, topk_ids, out, sort_order_out,
                            expert_ends_out, *bank.tensors())
-    if out is None:
-        out = torch.empty(T, H, dtype=hidden_states.dtype, device=dev)
-    p = _problem(hidden_states, topk_ids, topk_weights, bank.n_experts, bank.inter_size,
-                 bank.group_size, bank.n_shared)
-    L = _lib.lib()
-    ws = workspace if workspace is not None else _lib.workspace(
-        dev, L.exq_moe_workspace_size(p), "fused")
-    cb = bank.c_bank()
-    _lib.check(L.exq_moe_mixed_forward(
-        p, hidden_states.data_ptr(), topk_ids.data_ptr(), topk_weights.data_ptr(), cb,
-        out.data_ptr(), _lib.ptr(sort_order_out), _lib.ptr(expert_ends_out), ws.data_ptr(),
-        ws.numel(), _lib.stream_handle(dev)), "fused_experts_mixed")
-    return out
+    return _call(_lib.lib().exq_moe_mixed_forward, hidden_states, topk_ids, topk_weights,
+                 bank.n_experts, bank.inter_size, bank.n_shared, bank.group_size,
+                 (bank.c_bank(),), dev, out, sort_order_out, expert_ends_out, workspace,
+                 "fused_experts_mixed")

@@ -154,12 +154,14 @@ def routed_gemm(hidden: torch.Tensor, router_indices: torch.Tensor, n_experts: i
     if n <= _MAX_ROUTED_SLOTS:
         ids = router_indices.contiguous()
         dev = _lib.require_gpu(hidden, ids)
-        ws = _lib.workspace(dev, L.exq_moe_routed_gemm_workspace_size(n_tok, top_k, n_experts, K))
+        st = _lib.stream_handle(dev)
+        ws = _lib.workspace(dev, L.exq_moe_routed_gemm_workspace_size(n_tok, top_k, n_experts, K),
+                            stream=st)
         _lib.check(L.exq_moe_routed_gemm(
             hidden.data_ptr(), _lib.dtype_code(hidden.dtype), n_tok, K, ids.data_ptr(),
             _lib.dtype_code(ids.dtype), top_k, _lib.ptr(packed), _lib.ptr(scales),
             _lib.ptr(weights), n_experts, N, group_size, _lib.ptr(mask), out.data_ptr(),
-            ws.data_ptr(), ws.numel(), _lib.stream_handle(dev)), what)
+            ws.data_ptr(), ws.numel(), st), what)
         return
     dev = hidden.device
     ids = router_indices.reshape(-1).contiguous()
