@@ -62,11 +62,13 @@ __device__ __forceinline__ void gdma16(const void* p, unsigned char* lds) {
   __builtin_amdgcn_global_load_lds((gptr_t)p, (lptr_t)lds, 16, 0, 0);
 #endif
 }
-// The same through a buffer resource at voff + soff (soff wave-uniform).
+// The same through a buffer resource at voff + soff (soff wave-uniform); AUX 2:
+// nontemporal.
+template <int AUX = 0>
 __device__ __forceinline__ void bdma16(__amdgpu_buffer_rsrc_t r, unsigned char* lds, int voff,
                                        int soff) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lptr_t)lds, 16, voff, soff, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lptr_t)lds, 16, voff, soff, 0, AUX);
 #endif
 }
 
@@ -116,7 +118,7 @@ __device__ __forceinline__ uint4 deq_signed(uint32_t p, uint32_t mask, uint32_t 
 // contiguous range of units, 8 token groups x 8 weight tiles at a time, so
 // that the groups of one expert share its weights in that XCD's L2.
 __device__ __forceinline__ bool rows_unit(const GemmArgs& a, int t0, int n, int NT, int bid,
-                                          TgEntry& te, int& nt) {
+                                          TgEntry& te, int& nt, bool* once = nullptr) {
   const int U = ((n + 7) >> 3) * 8 * NT;
   const int per = (U + 7) >> 3;
   const int local = bid >> 3;
@@ -128,6 +130,9 @@ __device__ __forceinline__ bool rows_unit(const GemmArgs& a, int t0, int n, int 
   const int tgi = tb * 8 + (rem & 7);
   if (tgi >= n) return false;
   te = a.tg[t0 + tgi];
+  if (once)  // the expert's only group (an expert's groups are neighbours in the list)
+    *once = (tgi == 0 || a.tg[t0 + tgi - 1].e != te.e) &&
+            (tgi + 1 >= n || a.tg[t0 + tgi + 1].e != te.e);
   return te.cnt > 0;
 }
 
@@ -410,7 +415,12 @@ __global__ void __launch_bounds__(RTH, 4) rows_kernel(GemmArgs a, int n_tiles) {
 //
 // Bound: HBM, the weights of the active experts read once.  OLMoE shape (K =
 // 2048, 2048 weight rows) at 96 tokens: 115 us on the 128 x 128 tiles (whose
-// activation rows are mostly padding there) -> 107 us.
+// activation rows are mostly padding there) -> 107 us.  An expert with one token
+// group has its weights copied with the nontemporal hint, as only this work-group
+// reads them: the layer 196 -> 178 us (Qwen3 shape at 40 tokens 137 -> 126).
+// Weights that several groups share stay cached: the hint on them too cost 188 us
+// there and 244 -> 258 at 250 tokens.  The INT4 kernel's 64-byte row pieces are
+// half lines, and the hint loses the other half: 95 -> 105 us at 187 tokens.
 constexpr int WKC = 64;
 __device__ __forceinline__ int w_swz(int r) { return (r >> 1) & 7; }
 
@@ -424,8 +434,10 @@ __global__ void __launch_bounds__(RTH, 4) rows_bf16_kernel(GemmArgs a, int n_til
   constexpr int QB = TN / 32;  // weight copies per wave and chunk (8 rows each)
   TgEntry te;
   int nt;
-  if (!rows_unit(a, 0, a.hdr[2], n_tiles, blockIdx.x, te, nt)) return;  // BF16 groups
+  bool once;
+  if (!rows_unit(a, 0, a.hdr[2], n_tiles, blockIdx.x, te, nt, &once)) return;  // BF16 groups
   nt = uni_i(nt);
+  const bool nontemporal = uni_i(once ? 1 : 0) != 0;
   const int cnt = uni_i(te.cnt), pos0 = uni_i(te.pos0);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -453,8 +465,12 @@ __global__ void __launch_bounds__(RTH, 4) rows_bf16_kernel(GemmArgs a, int n_til
   auto copy = [&](unsigned char* A, unsigned char* B, int ch) {
     if (ch >= nch) return;
 #pragma unroll
-    for (int q = 0; q < QB; ++q)
-      bdma16(wr, B + (wave * QB + q) * 1024, vB[q], uni_i(ch * WKC * 2));
+    for (int q = 0; q < QB; ++q) {
+      if (nontemporal)
+        bdma16<2>(wr, B + (wave * QB + q) * 1024, vB[q], uni_i(ch * WKC * 2));
+      else
+        bdma16(wr, B + (wave * QB + q) * 1024, vB[q], uni_i(ch * WKC * 2));
+    }
     gdma16(pA + (int64_t)ch * WKC, A + wave * 1024);
   };
   f32x4_t acc[MT][NTW];

@@ -389,6 +389,30 @@ def test_routed_gemms(T, k, E, K, N, dtype, device):
     assert not out[n:].any() and not out[:ends[1]].any()
 
 
+@pytest.mark.parametrize("counts", [
+    [1], [33], [0, 32, 0, 33, 1],       # one group / two groups, alone and beside others
+    [31, 0, 64, 2, 65, 0, 1, 3],        # single-group experts between shared ones
+])
+def test_rows_gemm_group_counts(counts, device):
+    """Unquantised rows kernel: experts of one token group (weights copied
+    nontemporal) between experts of several; bf16 outputs of fp32 sums over K =
+    256 (one rounding, 2^-9 relative)."""
+    from exq_amd.kernels import moe_grouped_gemm
+    K, N = 256, 160
+    E = len(counts) + 8  # idle experts keep the average at or below 31 rows
+    banner(f"rows gemm groups {counts}")
+    rng = np.random.default_rng(sum(counts))
+    ids = rng.permutation(np.repeat(np.arange(len(counts)), counts))
+    x = torch.from_numpy(rng.standard_normal((ids.size, K)).astype(np.float32)).bfloat16()
+    w = torch.from_numpy((rng.standard_normal((E, N, K)) * 0.05).astype(np.float32)).bfloat16()
+    out = moe_grouped_gemm(x.to(device), w.to(device),
+                           torch.from_numpy(ids.reshape(-1, 1)).to(device), E)
+    order = np.argsort(ids, kind="stable")
+    ends = np.searchsorted(ids[order], np.arange(E + 1))
+    ref = moe.grouped_gemm_sorted(x.float().numpy()[order], w.float().numpy(), ends)
+    assert_close_rel(out, ref, TOL, f"rows gemm groups {counts}")
+
+
 @pytest.mark.parametrize("T,k,E", [(1, 1, 1), (40, 8, 64), (700, 4, 100), (1200, 4, 1023)])
 def test_unsort_output_routes(T, k, E, device):
     """unsort_output on the one-work-group sort and on the multi-block one, with
