@@ -20,14 +20,17 @@
 // groups), gate/up: 61 us; 39 us with only the copies left in, 46 us with only
 // the arithmetic.  Tiles of 16 or 64 rows, or of 256 weight rows, measured the
 // same or slower there (109 - 123 us a layer against 111), and so did weights
-// copied two chunks at a time in whole 128-byte lines (113).
+// copied two chunks at a time in whole 128-byte lines (113).  Three or four stages
+// instead of two, with three or two work-groups per CU: 95 -> 107 / 121 us (group
+// 64 at 48 tokens 67 -> 74 / 81): waves per SIMD hide more than copies in flight.
 //
 // Arithmetic.  Step s of a chunk covers k = 32 s .. 32 s + 31, so every step
 // lies inside one scale group: lane (r, q) of the MFMA 16x16x32 operands holds
 // k = 32 s + 8 q .. + 7 of row r (16 bytes of activations, one dword of packed
-// nibbles).  Nibbles become exact 16-bit floats of q - 8 (bf16: of (q - 8) / 16,
-// the 16 folded into the scale), a scale group's steps accumulate in fp32 and
-// the group's fp16 scale multiplies the sum in fp32.
+// nibbles), or another 8 k of the same scale group where a group holds several
+// steps.  Nibbles become exact 16-bit floats of q - 8 (bf16: of (q - 8) / 16, the
+// 16 folded into the scale), a scale group's steps accumulate in fp32 and the
+// group's fp16 scale multiplies the sum in fp32.
 #include "exq_internal.h"
 
 #include "dev_util.h"
@@ -140,9 +143,9 @@ __device__ __forceinline__ bool rows_unit(const GemmArgs& a, int t0, int n, int 
 // its multiples: a scale per chunk), with K % 128 == 0; 0: any group size and
 // any K % 32 == 0.
 template <bool BF, int MODE, int SPG>
-__device__ __forceinline__ void rows_body(const GemmArgs& a, int n_tiles, unsigned char* sA0,
-                                          unsigned char* sA1, unsigned char* sB0,
-                                          unsigned char* sB1) {
+__device__ __forceinline__ void rows_body(const GemmArgs& a, int n_tiles,
+                                          unsigned char* const (&sA)[2],
+                                          unsigned char* const (&sB)[2]) {
   constexpr int HN = TN / 2, HALF = NTW / 2;
   constexpr int QA = MT;        // activation copies per wave and chunk (4 rows each)
   constexpr int QB = NTW;       // weight copies per wave and chunk (16 rows each)
@@ -301,23 +304,53 @@ __device__ __forceinline__ void rows_body(const GemmArgs& a, int n_tiles, unsign
       }
     }
   };
-  // LDS reads of step s of chunk half hf: A at column 4 s + kq of row r16 (+ 4
-  // KiB per m-tile), B at column 4 hf + s, dword kq of weight row brow(t) + r16.
+  // LDS reads of step s: A at column 4 s + kq of row r16 (+ 4 KiB per m-tile), B
+  // at column s, dword kq of weight row brow(t) + r16.  Where a scale group holds
+  // several steps (group 64, multiples of 128) the order of k inside it is free,
+  // and a lane's weights for those steps are one read: k = 64 h + 16 kq + 8 j (step
+  // s = 2 h + j, 8 bytes) or k = 32 kq + 8 s (16 bytes), A read at the same k.  All
+  // these reads are free of bank conflicts under the maps above.  With the loop as
+  // one body per stage (fewer registers): Qwen3 shape at 187 tokens 98.4 -> 95.0 us
+  // a layer, Mixtral at 100 tokens 315 -> 308, group 96 at 64 tokens 75 -> 70.5,
+  // group 64 the same.
   const int asw = ra_swz(r16), bsw = rb_swz(r16);
   auto chunk = [&](const unsigned char* A, const unsigned char* B, int ch) {
+    uint32_t bw[NTW][4];
+    if constexpr (SPG == 4) {
+#pragma unroll
+      for (int t = 0; t < NTW; ++t) {
+        const uint4 v =
+            *reinterpret_cast<const uint4*>(B + (brow(t) + r16) * 64 + ((kq ^ bsw) * 16));
+        bw[t][0] = v.x, bw[t][1] = v.y, bw[t][2] = v.z, bw[t][3] = v.w;
+      }
+    } else if constexpr (SPG == 2) {
+#pragma unroll
+      for (int t = 0; t < NTW; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint2 v = *reinterpret_cast<const uint2*>(
+              B + (brow(t) + r16) * 64 + (((2 * h + (kq >> 1)) ^ bsw) * 16) + (kq & 1) * 8);
+          bw[t][2 * h] = v.x, bw[t][2 * h + 1] = v.y;
+        }
+    }
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       if (SPG == 0 && ch * 4 + s >= K / 32) break;  // wave-uniform: end of the contraction
       uint4 af[MT], bf[NTW];
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        af[mt] = *reinterpret_cast<const uint4*>(A + (mt * 16 + r16) * 256 +
-                                                 (((4 * s + kq) ^ asw) * 16));
+      for (int mt = 0; mt < MT; ++mt) {
+        const int col = SPG == 4   ? 4 * kq + s
+                        : SPG == 2 ? 8 * (s >> 1) + 2 * kq + (s & 1)
+                                   : 4 * s + kq;
+        af[mt] = *reinterpret_cast<const uint4*>(A + (mt * 16 + r16) * 256 + ((col ^ asw) * 16));
+      }
 #pragma unroll
-      for (int t = 0; t < NTW; ++t)
-        bf[t] = deq_signed<BF>(*reinterpret_cast<const uint32_t*>(B + (brow(t) + r16) * 64 +
-                                                                 ((s ^ bsw) * 16) + kq * 4),
-                               dq_mask, dq_magic);
+      for (int t = 0; t < NTW; ++t) {
+        if constexpr (SPG != 4 && SPG != 2)
+          bw[t][s] = *reinterpret_cast<const uint32_t*>(B + (brow(t) + r16) * 64 +
+                                                        ((s ^ bsw) * 16) + kq * 4);
+        bf[t] = deq_signed<BF>(bw[t][s], dq_mask, dq_magic);
+      }
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -347,22 +380,20 @@ __device__ __forceinline__ void rows_body(const GemmArgs& a, int n_tiles, unsign
   };
   load_window(sc0, sc1, 0);
   load_window(sn0, sn1, 1);
-  copy_a(sA0, 0);
-  copy_b(sB0, 0);
-  for (int ch = 0; ch < nch; ch += 2) {
-    barrier();
-    advance_window(ch);
-    copy_b(sB1, ch + 1);
-    copy_a(sA1, ch + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    chunk(sA0, sB0, ch);
-    if (ch + 1 >= nch) break;
-    barrier();
-    advance_window(ch + 1);
-    copy_b(sB0, ch + 2);
-    copy_a(sA0, ch + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    chunk(sA1, sB1, ch + 1);
+  copy_a(sA[0], 0);
+  copy_b(sB[0], 0);
+  for (int ch0 = 0; ch0 < nch; ch0 += 2) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {  // the stage is a constant in each copy of the body
+      const int ch = ch0 + i;
+      if (ch >= nch) break;
+      barrier();
+      advance_window(ch);
+      copy_b(sB[1 - i], ch + 1);
+      copy_a(sA[1 - i], ch + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      chunk(sA[i], sB[i], ch);
+    }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy outlives the work-group
 
@@ -403,7 +434,9 @@ __global__ void __launch_bounds__(RTH, 4) rows_kernel(GemmArgs a, int n_tiles) {
   __shared__ __attribute__((aligned(1024))) unsigned char sA1[MT * 4096];
   __shared__ __attribute__((aligned(1024))) unsigned char sB0[NTW * 4096];
   __shared__ __attribute__((aligned(1024))) unsigned char sB1[NTW * 4096];
-  rows_body<BF, MODE, SPG>(a, n_tiles, sA0, sA1, sB0, sB1);
+  unsigned char* const sA[2] = {sA0, sA1};
+  unsigned char* const sB[2] = {sB0, sB1};
+  rows_body<BF, MODE, SPG>(a, n_tiles, sA, sB);
 }
 
 // Unquantised weights: C = A x W^T with the same 32-row x 128-weight-row
