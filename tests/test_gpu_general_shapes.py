@@ -103,6 +103,32 @@ def test_rows_kernel_edges(H, I, g, dtype, device):
     assert_close_rel(out, ref, TOL, f"rows kernel H={H} I={I} g={g} {dtype}")
 
 
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 8, 9, 12, 16, 17])
+@pytest.mark.parametrize("H", [32, 96, 1056])
+def test_combine_slot_batches(k, H, device):
+    """Combine launch of the prefill and rows paths: slots in batches of 2, 4 or 8
+    with a short last one, columns past a block's end, dropped ids (no weight),
+    one token with none left."""
+    from exq_amd.kernels import fused_experts
+    banner(f"combine k={k} H={H}")
+    E, T, I, g = 20, 11, 64, 32
+    p13, s13 = _bank(E, 2 * I, H, g, H + k, device)
+    p2, s2 = _bank(E, H, I, g, H + k + 1, device)
+    rng = np.random.default_rng(100 * k + H)
+    ids = np.stack([rng.choice(E, size=k, replace=False) for _ in range(T)]).astype(np.int64)
+    ids[rng.random((T, k)) < 0.2] = -1
+    ids[3] = -1
+    w = rng.random((T, k)).astype(np.float32)
+    x = torch.from_numpy(synth.hidden_np(T, H, 5)).to(torch.bfloat16).to(device)
+    out = fused_experts(x, p13, s13, p2, s2, torch.from_numpy(w).to(device),
+                        torch.from_numpy(ids).to(device))
+    # the oracle's dropped slots: any expert, weight 0
+    ref = oracle_int4_layer(x, p13, s13, p2, s2, np.maximum(ids, 0),
+                            np.where(ids < 0, 0, w).astype(np.float32))
+    assert_close_rel(out, ref, TOL, f"combine k={k} H={H}")
+    assert not out[3].any()
+
+
 def test_general_shape_rejections(device):
     from exq_amd import _lib
     from exq_amd.kernels import MixedExpertBank, fused_experts, fused_experts_mixed, \
