@@ -5,6 +5,7 @@
 #include <type_traits>
 
 #include "exq_common.h"
+#include "unit_order.h"
 
 namespace exq {
 
@@ -104,9 +105,10 @@ int launch_tile_gemm(int tier, int mode, bool bf, const GemmArgs& a, const float
 // The tiles of one projection in one launch (tile_mix_kernel): 128 x 256
 // scaled-operand INT4 tiles over token groups [hdr[1], hdr[3]), 128 x 256 INT8
 // tiles over [hdr[2], hdr[1]), 64 x 256 INT4 tiles over [hdr[3], hdr[0]) (row
-// sums from launch_group_rowsum), then BF16 tiles over [0, hdr[2]).  cap_* bound each range's token groups (0: the range
-// is empty); the grid is sized from them and each range's real size is read
-// on the device.
+// sums from launch_group_rowsum), then BF16 tiles over [0, hdr[2]).  cap_* bound
+// each range's token groups; 0 leaves the range out, also where the list holds
+// such groups (they are another kernel's).  The grid is sized from them and each
+// range's real size is read on the device.
 int launch_tile_mix(int mode, bool bf, const GemmArgs& a, const float* rs, int64_t rs_rows,
                     int64_t x_bytes, int64_t cap_ps, int64_t cap_i8, int64_t cap_64,
                     int64_t cap_bf, hipStream_t s);

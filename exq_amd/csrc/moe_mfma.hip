@@ -364,8 +364,8 @@ __global__ void __launch_bounds__(NTH, 2) moe_gemm_kernel(GemmArgs a) {
   // XCD-aware order: work-group i runs on XCD i % 8, so each XCD takes a
   // contiguous range of units and neighbouring blocks of one token group
   // (which share the staged activations) stay in one L2.
-  // A grid smaller than 8 * per (when only the INT8 groups are left here)
-  // strides over the order.
+  // A grid smaller than 8 * per (when the tiles take some of the tiers) strides
+  // over the order.
   const int per = (U + 7) >> 3;
   for (int idx = blockIdx.x; idx < 8 * per; idx += gridDim.x) {
     const int local = idx >> 3;
@@ -441,8 +441,10 @@ __global__ void __launch_bounds__(256) combine_partials_kernel(
 template <int MODE>
 int launch_gemm(bool bf, const GemmArgs& a, int64_t units_cap, hipStream_t s) {
   int64_t grid = 8 * cdiv(units_cap, 8);
-  // With the tiled kernels running, only INT8 groups (if any) are left here:
-  // a resident-sized grid strides over them instead of launching the cap.
+  // With the tiled kernels running, at most the tiers that their tiles do not
+  // take are left here (INT4 of a group size other than 128, INT8 where the
+  // 256-row tiles do not divide the weights): a resident-sized grid strides over
+  // them instead of launching the cap.
   if ((a.skip_i4 || a.skip_bf) && grid > 2048) grid = 2048;
   if (grid <= 0) return EXQ_SUCCESS;
   if (grid > INT32_MAX)
@@ -593,9 +595,9 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
   rp.ends = reinterpret_cast<int*>(ws + L.ends);
   rp.sorted = reinterpret_cast<int*>(ws + L.sorted);
   rp.tg = reinterpret_cast<TgEntry*>(ws + L.tg);
-  // INT4 and BF16 experts run on the tiled kernels (128- or 64-row token
-  // groups) when both projections fit them and the gathered activations are 32-bit
-  // addressable; INT8 experts (and everything else) on the grouped kernel.
+  // The experts of each tier run on the tiled kernels (128- or 64-row token
+  // groups) when both projections fit that tier's tiles and the gathered
+  // activations are 32-bit addressable, on the grouped kernel otherwise.
   const int gs = (int)p->group_size;
   // all-INT4 layers of other shapes or few rows per expert: routing plan + rows
   // kernels + combine

@@ -1249,18 +1249,14 @@ __global__ void __launch_bounds__(TT, 2) tile_gemm_bf16_kernel(GemmArgs a, TileA
   tile_gemm_bf16_body<BF, MODE>(a, ta, blockIdx.x, sA0, sA1, sB0, sB1);
 }
 
-// Work-groups of tile_unit's unit range over n token groups (a multiple of
-// eight groups times the weight tiles per group).
-__device__ __forceinline__ int tile_unit_count(int n, int n_tiles) {
-  return ((n + 7) >> 3) * 8 * n_tiles;
-}
-
 // The tiles of one projection in one grid, in four ranges whose sizes come
 // from the token-group list on the device: 128 x 256 scaled-operand INT4 tiles
 // over the big-group INT4 experts [hdr[1], hdr[3]), 128 x 256 INT8 tiles over
 // [hdr[2], hdr[1]), 64 x 256 INT4 tiles over the other INT4 experts [hdr[3],
 // hdr[0]), then BF16 tiles over [0, hdr[2]).  All take 16 KiB per operand
-// stage, so the LDS is shared.  The host sizes the grid from upper bounds;
+// stage, so the LDS is shared.  A range that is not part of the launch has no
+// weight tiles and so no units, whatever the list holds there (mix_tiles).  The
+// host sizes the grid from upper bounds;
 // the work-groups past the four ranges return at once, after every real unit
 // in dispatch order.  The longest units (the 128-row tiles) go first and the
 // BF16 units fill the last, partly empty round of the others
@@ -1277,19 +1273,19 @@ __global__ void __launch_bounds__(TT, 2) tile_mix_kernel(GemmArgs a, TileArgs tp
   __shared__ __attribute__((aligned(1024))) unsigned char sB0[AB_STAGE];
   __shared__ __attribute__((aligned(1024))) unsigned char sB1[AB_STAGE];
   int bid = (int)blockIdx.x;
-  const int u_ps = tile_unit_count(a.hdr[3] - a.hdr[1], tps.n_tiles);
+  const int u_ps = unit_count(a.hdr[3] - a.hdr[1], tps.n_tiles);
   if (bid < u_ps) {
     tile_ps_body<BF, MODE>(a, tps, bid, sA0, sA1, sB0, sB1);
     return;
   }
   bid -= u_ps;
-  const int u_i8 = tile_unit_count(a.hdr[1] - a.hdr[2], ti8.n_tiles);
+  const int u_i8 = unit_count(a.hdr[1] - a.hdr[2], ti8.n_tiles);
   if (bid < u_i8) {
     tile_i8_body<BF, MODE>(a, ti8, bid, sA0, sA1, sB0, sB1);
     return;
   }
   bid -= u_i8;
-  const int u_64 = tile_unit_count(a.hdr[0] - a.hdr[3], t64.n_tiles);
+  const int u_64 = unit_count(a.hdr[0] - a.hdr[3], t64.n_tiles);
   if (bid < u_64) {
     tile_gemm_body<BF, MODE, 4, 4>(a, t64, bid, sA0, sA1, sB0, sB1);
     return;
@@ -1421,14 +1417,18 @@ int launch_tile_mix(int mode, bool bf, const GemmArgs& a, const float* rs, int64
   tps.rs = nullptr;  // scaled weight operands: no row sums
   tps.rs_rows = 0;
   tps.x_bytes = x_bytes;
-  tps.n_tiles = mode == MODE_GATEUP ? a.inter / 128 : a.n_rows / 256;  // 256-row INT4 tiles
+  const MixTiles t = mode == MODE_GATEUP
+                         ? mix_tiles(a.inter / 128, a.inter / 64, cap_ps, cap_i8, cap_64, cap_bf)
+                         : mix_tiles(a.n_rows / 256, a.n_rows / 128, cap_ps, cap_i8, cap_64, cap_bf);
+  tps.n_tiles = t.ps;
   tps.h_lo = 1;
   tps.h_hi = 3;
   ti8 = tps;
-  ti8.n_tiles = cap_i8 > 0 ? tps.n_tiles : 0;
+  ti8.n_tiles = t.i8;
   ti8.h_lo = 2;
   ti8.h_hi = 1;
   t64 = tps;
+  t64.n_tiles = t.t64;
   t64.rs = rs;
   t64.rs_rows = (int)rs_rows;
   t64.h_lo = 3;
@@ -1436,11 +1436,10 @@ int launch_tile_mix(int mode, bool bf, const GemmArgs& a, const float* rs, int64
   tbf.rs = nullptr;
   tbf.rs_rows = 0;
   tbf.x_bytes = x_bytes;
-  tbf.n_tiles = cap_bf > 0 ? (mode == MODE_GATEUP ? a.inter / 64 : a.n_rows / 128) : 0;
+  tbf.n_tiles = t.bf;
   tbf.h_lo = 0;
   tbf.h_hi = 2;
-  const int64_t grid = 8 * cdiv(cap_ps, 8) * tps.n_tiles + 8 * cdiv(cap_i8, 8) * ti8.n_tiles +
-                       8 * cdiv(cap_64, 8) * t64.n_tiles + 8 * cdiv(cap_bf, 8) * tbf.n_tiles;
+  const int64_t grid = mix_grid(t, cap_ps, cap_i8, cap_64, cap_bf);
   if (grid <= 0) return EXQ_SUCCESS;
   if (grid > INT32_MAX || rs_rows > INT32_MAX)
     return set_error(EXQ_ERROR_UNSUPPORTED, "tile_mix: problem too large");

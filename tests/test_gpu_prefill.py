@@ -273,6 +273,29 @@ def test_prefill_int8_tiles(H, I, tiers, act, device):
     assert_close_rel(out, _oracle(bank, x, ids, w), TOL, f"prefill int8 tiles {H} {I} {act}")
 
 
+@pytest.mark.parametrize("H,I,g,T", [
+    (512, 256, 256, 65), (512, 256, 256, 330),
+    (768, 384, 384, 5),      # a group size that the decode kernels do not take
+    (768, 384, 384, 65), (768, 384, 384, 330),
+])
+@pytest.mark.parametrize("tiers", [[1, 1, 2, 2, 1, 2, 2, 2], [1, 0, 2, 2, 1, 0, 2, 2]])
+@pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
+def test_prefill_int8_tiles_other_groups(H, I, g, T, tiers, act, device):
+    """INT8 (and BF16) experts on the tiles beside INT4 experts whose group size
+    keeps them on the grouped kernel: the tile launch has no INT4 units."""
+    from exq_amd.kernels import MixedExpertBank, fused_experts_mixed
+    from tests.test_gpu_mixed import _oracle
+    banner(f"prefill int8 tiles H={H} I={I} g={g} T={T} {tiers} {act}")
+    cfg = synth.MoeConfig("int8_groups", 57, H, I, len(tiers), 2, False)
+    w13, w2 = synth.expert_weights_gpu(len(tiers), I, H, 995 + g, device)
+    bank = MixedExpertBank.from_weights(w13, w2, tiers, act_dtype=act, group_size=g)
+    ids, w = synth.routing(cfg, T)
+    x = _hidden(T, H, 996, device, act)
+    out = fused_experts_mixed(x, bank, torch.from_numpy(w).to(device),
+                              torch.from_numpy(ids).to(device))
+    assert_close_rel(out, _oracle(bank, x, ids, w), TOL, f"prefill int8 tiles g={g} T={T} {act}")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_prefill_sorted_bf16_gemm_tiled(dtype, device):
     """Unquantised sorted-row GEMM with N % 128 == 0 runs on the BF16 tiled
