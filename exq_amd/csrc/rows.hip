@@ -224,12 +224,15 @@ __device__ __forceinline__ void rows_body(const GemmArgs& a, int n_tiles,
       gdma16(pA[q] + (int64_t)ch * RKC - (in ? 0 : cA[q]), A + (wave * QA + q) * 1024);
     }
   };
+  // (No copy or load here has a scalar offset at or past its resource's end: the
+  // range check of the lanes' offsets against size - scalar offset would be
+  // against a negative number.)
   auto copy_b = [&](unsigned char* B, int ch) {
+    if (ch >= nch) return;
 #pragma unroll
     for (int q = 0; q < QB; ++q) {
-      // past the row's end (a short last chunk, or a whole one: every chunk
-      // issues its copies): nothing to fetch
-      const int v = (SPG != 0 ? ch < nch : ch * RKC + cB[q] * 32 < K) ? vB[q] : OOB_OFF;
+      // past the row's end in a short last chunk: nothing to fetch
+      const int v = SPG != 0 || ch * RKC + cB[q] * 32 < K ? vB[q] : OOB_OFF;
       bdma16(wr, B + (wave * QB + q) * 1024, v, uni_i(ch * (RKC / 2)));
     }
   };
@@ -246,13 +249,15 @@ __device__ __forceinline__ void rows_body(const GemmArgs& a, int n_tiles,
   uint32_t sc0[NTW], sc1[NTW], sn0[NTW], sn1[NTW];  // this window's and the next one's dwords
   int win = 0;
   auto load_window = [&](uint32_t (&d0)[NTW], uint32_t (&d1)[NTW], int w) {
+    // a window past the row's last group (never used) reads window 0 again
+    const int off = uni_i(w * 16 < ngs ? w * 32 : 0);
 #pragma unroll
     for (int t = 0; t < NTW; ++t) {
       const __amdgpu_buffer_rsrc_t sr = MODE == MODE_GATEUP && t >= HALF ? su : sg;
-      const uint32_t h0 = __builtin_amdgcn_raw_buffer_load_b16(sr, vS[t], uni_i(w * 32), 0);
-      const uint32_t h1 = __builtin_amdgcn_raw_buffer_load_b16(sr, vS[t] + 2, uni_i(w * 32), 0);
-      const uint32_t h2 = __builtin_amdgcn_raw_buffer_load_b16(sr, vS[t] + 4, uni_i(w * 32), 0);
-      const uint32_t h3 = __builtin_amdgcn_raw_buffer_load_b16(sr, vS[t] + 6, uni_i(w * 32), 0);
+      const uint32_t h0 = __builtin_amdgcn_raw_buffer_load_b16(sr, vS[t], off, 0);
+      const uint32_t h1 = __builtin_amdgcn_raw_buffer_load_b16(sr, vS[t] + 2, off, 0);
+      const uint32_t h2 = __builtin_amdgcn_raw_buffer_load_b16(sr, vS[t] + 4, off, 0);
+      const uint32_t h3 = __builtin_amdgcn_raw_buffer_load_b16(sr, vS[t] + 6, off, 0);
       d0[t] = h0 | (h1 << 16);
       d1[t] = h2 | (h3 << 16);
     }
@@ -367,11 +372,10 @@ __device__ __forceinline__ void rows_body(const GemmArgs& a, int n_tiles,
     }
   };
 
-  // The wave's copies of the chunk have landed when at most the next pair's QB
-  // weight copies (issued after them) are outstanding; then every wave's have,
-  // and every wave has finished reading what is overwritten next.
-  // (the builtin waits are known to the compiler's own wait insertion, which
-  // otherwise waits for every pending copy at the chunk's first LDS read)
+  // Every copy of this wave has landed and its LDS reads are done; behind the
+  // barrier every wave's are, and what they read may be overwritten.  (The
+  // builtin wait is known to the compiler's own wait insertion, which otherwise
+  // waits again at the chunk's first LDS read.)
   auto barrier = [&]() {
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
     asm volatile("" ::: "memory");
@@ -591,7 +595,6 @@ bool general_shape(int64_t K, int64_t group_size) {
   return K >= 32 && K % 32 == 0 && group_size >= 32 && group_size % 32 == 0 &&
          K % group_size == 0;
 }
-
 
 int launch_rows_gemm(int mode, bool bf, const GemmArgs& a, int64_t tg_cap, hipStream_t s) {
   if (a.K > (1 << 24))  // 32-bit offsets inside a tile's weight rows

@@ -103,6 +103,35 @@ def test_rows_kernel_edges(H, I, g, dtype, device):
     assert_close_rel(out, ref, TOL, f"rows kernel H={H} I={I} g={g} {dtype}")
 
 
+@pytest.mark.parametrize("K,N,g", [
+    (32, 1, 32),        # one weight row of one scale group
+    (160, 129, 32),     # K % 128 = 32: the last tile is one row whose last chunk is short
+    (224, 257, 32),     # K % 128 = 96
+    (640, 130, 32),     # 20 groups a row: two 16-group scale windows of two rows
+    (544, 1, 32),       # 17 groups: the second window is one group
+    (96, 129, 96),
+    (1024, 129, 64),    # whole chunks, one row in the last tile
+    (512, 1, 256),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rows_kernel_last_weight_row(K, N, g, dtype, device):
+    """Tiles of one or two weight rows at the end of the packed weights and scales:
+    chunks and scale windows past a row's end are past the resource too."""
+    from exq_amd.kernels import moe_int4_forward
+    banner(f"rows kernel K={K} N={N} g={g} {dtype}")
+    E, T = 3, 41
+    p, s = _bank(E, N, K, g, K + N, device)
+    rng = np.random.default_rng(K + N)
+    ids = rng.integers(0, E, (T, 1))
+    x = torch.from_numpy(rng.standard_normal((T, K)).astype(np.float32)).to(dtype).to(device)
+    out = moe_int4_forward(x, p, s, torch.from_numpy(ids).to(device), E)
+    order = np.argsort(ids[:, 0], kind="stable")
+    ends = np.searchsorted(ids[order, 0], np.arange(E + 1))
+    ref = moe.grouped_gemm_sorted(x.float().cpu().numpy()[order],
+                                  quant.dequant_int4(p.cpu().numpy(), s.cpu().numpy()), ends)
+    assert_close_rel(out, ref, TOL, f"rows kernel K={K} N={N} g={g} {dtype}")
+
+
 @pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 8, 9, 12, 16, 17])
 @pytest.mark.parametrize("H", [32, 96, 1056])
 def test_combine_slot_batches(k, H, device):
