@@ -20,6 +20,8 @@
 // exactly once per token group; activations are staged in LDS per wave.
 #include "exq_internal.h"
 
+#include "dev_util.h"
+
 namespace exq {
 namespace {
 
@@ -388,44 +390,73 @@ __global__ void __launch_bounds__(NTH, 2) moe_gemm_kernel(GemmArgs a) {
 // out[t, h] = sum_j w[t, j] * partial[t*kp + j, h] over the routed slots that
 // were not dropped (shared-expert slots j >= k have weight 1), fp32 in the
 // fixed order j = 0..kp-1, rounded once to the activation dtype.  One thread
-// per 4 consecutive h of one token (block b: token b / nbx), so that the routing
-// entries are scalar loads and the rows of JB slots are in flight at once.
-// Against one row at a time behind its id, layer: group 64 at 3 tokens 38.5 ->
-// 37.1 us, at 48 tokens 66.2 -> 65.0, Qwen3 shape at 187 tokens 96.1 -> 94.0,
-// DeepSeek-V2-Lite at 2048 tokens (142 MB, at the HBM's rate) 447.3 -> 442.3.
-// A separate launch: the kernel boundary makes every
-// partial row visible without a device-wide fence in the down kernel.
+// per 4 consecutive h of one token (grid: tokens x column blocks), so that the
+// routing entries are scalar loads, all of a batch of JB slots in flight, and
+// then the rows of the slots that were not dropped.  Bound: bytes.  Against one
+// row at a time behind its id, layer: group 64 at 48 tokens 66.2 -> 64.1 us, Qwen3
+// shape at 187 tokens 96.1 -> 93.5; with 7 of 8 ids dropped (a rank that holds an
+// eighth of the experts), Qwen3 shape at 4096 tokens 128 -> 122.  Fetching the rows
+// without waiting for the ids is 0.5 % of a large layer faster (DeepSeek-V2-Lite
+// at 2048 tokens 455.3 -> 452.9) where no id is dropped, and reads eight times the
+// bytes on that rank: 151 us.
+// A separate launch: the kernel boundary makes every partial row visible without
+// a device-wide fence in the down kernel.
 template <bool BF, int JB>
 __global__ void __launch_bounds__(256) combine_partials_kernel(
     const float* __restrict__ part, const void* __restrict__ ids, int ids_dtype,
-    const void* __restrict__ topk_w, int w_dtype, int nbx, int k, int kp, int E, int H,
+    const void* __restrict__ topk_w, int w_dtype, int k, int kp, int E, int H,
     uint16_t* __restrict__ out) {
-  const int t = (int)(blockIdx.x / (uint32_t)nbx);
-  const int hq = (int)(blockIdx.x - (uint32_t)t * nbx) * blockDim.x + threadIdx.x;
+  const int t = blockIdx.x;
+  const int hq = blockIdx.y * blockDim.x + threadIdx.x;
   if (hq >= H >> 2) return;
   const int h = hq * 4;
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  const float* row = part + (int64_t)t * kp * H + h;
+  const int64_t slot0 = (int64_t)t * k;
+  const int id64 = ids_dtype == EXQ_DTYPE_I64 ? 1 : 0;
+  const uint32_t* id32 = reinterpret_cast<const uint32_t*>(ids);
   for (int j0 = 0; j0 < kp; j0 += JB) {
     float4 pv[JB];
     float wgt[JB];
-    bool use[JB];
+    // the routing entries of the batch, all in flight (slots past k repeat the last)
+    uint32_t lo[JB], hi[JB];
 #pragma unroll
     for (int q = 0; q < JB; ++q) {
-      const int j = j0 + q;
-      // slots past the last repeat it; rows of dropped ids are read, not used
-      pv[q] = *reinterpret_cast<const float4*>(row + (int64_t)(j < kp ? j : kp - 1) * H);
-      wgt[q] = 1.f;
-      use[q] = j < kp;
-      if (j < k) {
-        const int64_t id = load_index(ids, ids_dtype, (int64_t)t * k + j);
-        use[q] = id >= 0 && id < E;
-        wgt[q] = load_as_f32(topk_w, w_dtype, (int64_t)t * k + j);
+      const int64_t i = (slot0 + (j0 + q < k ? j0 + q : k - 1)) << id64;
+      lo[q] = id32[i];
+      hi[q] = id32[i + id64];
+    }
+    if (w_dtype == EXQ_DTYPE_F32) {
+      const float* w = reinterpret_cast<const float*>(topk_w) + slot0;
+#pragma unroll
+      for (int q = 0; q < JB; ++q) wgt[q] = w[j0 + q < k ? j0 + q : k - 1];
+    } else {
+      const uint16_t* w = reinterpret_cast<const uint16_t*>(topk_w) + slot0;
+#pragma unroll
+      for (int q = 0; q < JB; ++q) {
+        const uint32_t b = w[j0 + q < k ? j0 + q : k - 1];
+        wgt[q] = w_dtype == EXQ_DTYPE_BF16 ? bf16_bits_to_f32(b) : f16_bits_to_f32(b);
       }
+    }
+    // rows of dropped ids are not fetched: an offset past the batch's rows reads 0,
+    // and their weight is 0 whatever the caller left there
+    const int left = kp - j0 < JB ? kp - j0 : JB;
+    const __amdgpu_buffer_rsrc_t rows =
+        dev::make_rsrc(part + ((int64_t)t * kp + j0) * H, (int64_t)left * H * 4);
+#pragma unroll
+    for (int q = 0; q < JB; ++q) {
+      // (all-ones masks and no conditions: scalar arithmetic, one row load each)
+      const int j = j0 + q;
+      const uint32_t h32 = hi[q] & (uint32_t)-id64;
+      const int out_of = (int)(lo[q] | ((uint32_t)(E - 1) - lo[q]) | h32 | (0u - h32)) >> 31;
+      const int shared = (k - 1 - j) >> 31, past = (kp - 1 - j) >> 31;
+      const int drop = (out_of & ~shared) | past;
+      const int off = (q * H * 4 & ~drop) | (dev::OOB_OFF & drop);
+      pv[q] = __builtin_bit_cast(float4,
+                                 __builtin_amdgcn_raw_buffer_load_b128(rows, off + h * 4, 0, 0));
+      wgt[q] = __int_as_float(((__float_as_int(wgt[q]) & ~shared) | (0x3f800000 & shared)) & ~drop);
     }
 #pragma unroll
     for (int q = 0; q < JB; ++q) {
-      if (!use[q]) continue;
       acc[0] += wgt[q] * pv[q].x;
       acc[1] += wgt[q] * pv[q].y;
       acc[2] += wgt[q] * pv[q].z;
@@ -827,14 +858,14 @@ int fused_forward_impl(const exq_moe_problem* p, const void* hidden, const void*
       if (st) return st;
     }
   }
-  const int nbx = (int)cdiv(H / 4, 256);
-  const dim3 cgrid((unsigned)((int64_t)T * nbx));
+  const int nbx = (int)cdiv(H / 4, T < (1 << 24) ? 256 : 128);  // T * block below 2^32 threads
+  const dim3 cgrid((unsigned)T, (unsigned)nbx);
   const dim3 cblock((unsigned)(64 * cdiv(H / 4, 64 * (int64_t)nbx)));
   // rows in flight: as few spare loads in the last batch as the slot count allows
   auto combine = [&](auto bfc, auto jb) {
     hipLaunchKernelGGL((combine_partials_kernel<decltype(bfc)::value, decltype(jb)::value>), cgrid,
                        cblock, 0, s, reinterpret_cast<const float*>(ws + L.partial), topk_ids,
-                       p->ids_dtype, topk_weights, p->weights_dtype, nbx, k, kp, E, H,
+                       p->ids_dtype, topk_weights, p->weights_dtype, k, kp, E, H,
                        reinterpret_cast<uint16_t*>(out));
   };
   auto combine_act = [&](auto bfc) {

@@ -158,6 +158,33 @@ def test_combine_slot_batches(k, H, device):
     assert not out[3].any()
 
 
+@pytest.mark.parametrize("ids_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("w_dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("k", [3, 8, 9])
+def test_combine_dropped_slots(k, w_dtype, ids_dtype, device):
+    """Rows of dropped ids are neither fetched nor weighted: -1, E, (64-bit) an id
+    whose low word is in range, each with a NaN or infinite weight."""
+    from exq_amd.kernels import fused_experts
+    banner(f"combine dropped k={k} {w_dtype} {ids_dtype}")
+    E, T, H, I, g = 16, 33, 160, 64, 32
+    p13, s13 = _bank(E, 2 * I, H, g, 900 + k, device)
+    p2, s2 = _bank(E, H, I, g, 901 + k, device)
+    rng = np.random.default_rng(k)
+    good = np.stack([rng.choice(E, size=k, replace=False) for _ in range(T)]).astype(np.int64)
+    w = torch.from_numpy(rng.random((T, k)).astype(np.float32)).to(w_dtype)
+    drop = rng.random((T, k)) < 0.6
+    bad = [-1, E] + ([2**32 + 3, -2**32 + 3] if ids_dtype == torch.int64 else [])
+    ids = np.where(drop, rng.choice(np.array(bad), (T, k)), good)
+    ref_w = np.where(drop, 0, w.float().numpy()).astype(np.float32)
+    w[torch.from_numpy(drop)] = float("nan")
+    w[0][torch.from_numpy(drop[0])] = float("inf")
+    x = torch.from_numpy(synth.hidden_np(T, H, 6)).to(torch.bfloat16).to(device)
+    out = fused_experts(x, p13, s13, p2, s2, w.to(device),
+                        torch.from_numpy(ids).to(ids_dtype).to(device))
+    ref = oracle_int4_layer(x, p13, s13, p2, s2, good, ref_w)
+    assert_close_rel(out, ref, TOL, f"combine dropped k={k} {w_dtype} {ids_dtype}")
+
+
 def test_general_shape_rejections(device):
     from exq_amd import _lib
     from exq_amd.kernels import MixedExpertBank, fused_experts, fused_experts_mixed, \
