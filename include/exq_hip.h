@@ -216,7 +216,10 @@ int exq_moe_grouped_gemm(const void* a_sorted, int act_dtype, int64_t n_rows, in
  * expert e), rows of ids outside [0, n_experts) and of experts with a zero
  * expert_mask entry left unwritten.  The rows are gathered by the GEMM.  INT4
  * weights (packed, scales) or unquantised ones (weights, with packed and scales
- * null), shapes as above; n_tokens * top_k <= 2^24.  Replaces the launch
+ * null), shapes as above; n_tokens * top_k <= 2^24.  Past 2 GiB of hidden the
+ * tiles cannot address it: such calls run on the rows kernels, and sorting and
+ * gathering first (exq_dispatch, exq_gather_hidden, the sorted-row GEMMs) is the
+ * faster sequence unless experts have few rows.  Replaces the launch
  * sequences of moe_int4_forward and moe_grouped_gemm
  * (exq/kernels/moe_int4_kernel.py:245-327, moe_grouped_gemm.py:173-227).
  */

@@ -412,6 +412,31 @@ def test_routed_gemms(T, k, E, K, N, dtype, device):
     assert not out[n:].any() and not out[:ends[1]].any()
 
 
+def test_routed_gemms_past_two_gib_of_tokens(device):
+    """More token bytes than the tiles address from the routing: sorted and gathered first."""
+    from exq_amd.kernels import moe_grouped_gemm, moe_int4_forward, pack_experts_int4
+    banner("routed gemms past 2 GiB")
+    T, K, N, E = (1 << 17) + 37, 8192, 128, 2
+    rng = np.random.default_rng(5)
+    ids = rng.integers(0, E, (T, 1))
+    gen = torch.Generator(device=device).manual_seed(6)
+    x = torch.randn(T, K, generator=gen, device=device, dtype=torch.bfloat16)
+    w = (torch.randn(E, N, K, generator=gen, device=device) * 0.02).to(torch.bfloat16)
+    tid = torch.from_numpy(ids).to(device)
+    order = np.argsort(ids[:, 0], kind="stable")
+    cut = int((ids == 0).sum())
+    rows = np.unique(np.r_[0, 1, cut - 1, cut, T - 1, rng.integers(0, T, 40)])
+    a = x[torch.from_numpy(order[rows]).to(device)].float().cpu().numpy()
+    ends = np.array([0, int((rows < cut).sum()), rows.size])
+    p, s = pack_experts_int4(w.to(torch.float16), 128)
+    for name, out, ref_w in (
+            ("int4", moe_int4_forward(x, p, s, tid, E),
+             quant.dequant_int4(p.cpu().numpy(), s.cpu().numpy())),
+            ("full", moe_grouped_gemm(x, w, tid, E), w.float().cpu().numpy())):
+        got = out[torch.from_numpy(rows).to(device)]
+        assert_close_rel(got, moe.grouped_gemm_sorted(a, ref_w, ends), TOL, f"past 2 GiB {name}")
+
+
 @pytest.mark.parametrize("counts", [
     [1], [33], [0, 32, 0, 33, 1],       # one group / two groups, alone and beside others
     [31, 0, 64, 2, 65, 0, 1, 3],        # single-group experts between shared ones

@@ -314,3 +314,40 @@ def test_mixed_bank_checks_tier_and_index_values():
         with pytest.raises(ValueError, match=msg):
             MixedExpertBank(tier=torch.tensor(tier, dtype=torch.int8),
                             index=torch.tensor(index, dtype=torch.int32), **kw)
+
+
+@pytest.mark.parametrize("n_tok,k,K,routed", [
+    (1, 8, 2048, True), ((1 << 18) - 1, 1, 4096, True), (1 << 18, 1, 4096, False),
+    (300000, 2, 4096, False), (1 << 23, 2, 64, True), ((1 << 23) + 1, 2, 64, False),
+])
+@pytest.mark.parametrize("int4", [True, False])
+def test_routed_gemm_sorts_and_gathers_past_its_limits(monkeypatch, n_tok, k, K, routed, int4):
+    """Up to 2^24 slots and 2 GiB of tokens the GEMM gathers its rows itself; past either, the
+    sort, the gathered copy and the sorted-row GEMM on tiles."""
+    from exq_amd import _lib
+    from exq_amd.kernels import moe_int4_kernel as m
+    calls = []
+
+    class Recorder:
+        def __getattr__(self, name):
+            def entry(*a):
+                calls.append(name)
+                return 0
+            return entry
+
+    monkeypatch.setattr(_lib, "lib", lambda: Recorder())
+    monkeypatch.setattr(_lib, "require_gpu", lambda *t: torch.device("meta"))
+    monkeypatch.setattr(_lib, "stream_handle", lambda dev: 0)
+    monkeypatch.setattr(_lib, "workspace", lambda *a, **kw: torch.empty(0, dtype=torch.uint8))
+    monkeypatch.setattr(m, "dispatch", lambda *a: calls.append("dispatch"))
+    monkeypatch.setattr(m, "gather_hidden", lambda *a: calls.append("gather"))
+    x = torch.empty(n_tok, K, dtype=torch.bfloat16, device="meta")
+    ids = torch.empty(n_tok, k, dtype=torch.int64, device="meta")
+    w = torch.empty(2, 128, K // 2 if int4 else K, device="meta",
+                    dtype=torch.uint8 if int4 else torch.bfloat16)
+    s = torch.empty(2, 128, 1, dtype=torch.float16, device="meta")
+    out = torch.empty(n_tok * k, 128, dtype=torch.bfloat16, device="meta")
+    m.routed_gemm(x, ids, 2, 128, K, out, **(dict(packed=w, scales=s) if int4 else dict(weights=w)))
+    sorted_gemm = "exq_moe_int4_gemm" if int4 else "exq_moe_grouped_gemm"
+    assert ("exq_moe_routed_gemm" in calls) == routed
+    assert ("gather" in calls, sorted_gemm in calls) == (not routed, not routed)
