@@ -116,22 +116,12 @@ __device__ __forceinline__ uint4 deq_signed(uint32_t p, uint32_t mask, uint32_t 
   return o;
 }
 
-// Unit (token group, weight tile) of work-group bid over n token groups from
-// t0, in XCD-aware order (work-group i runs on XCD i % 8): each XCD takes a
-// contiguous range of units, 8 token groups x 8 weight tiles at a time, so
-// that the groups of one expert share its weights in that XCD's L2.
+// Unit (token group, weight tile) of work-group bid over n token groups from t0
+// (unit_order.h).
 __device__ __forceinline__ bool rows_unit(const GemmArgs& a, int t0, int n, int NT, int bid,
                                           TgEntry& te, int& nt, bool* once = nullptr) {
-  const int U = ((n + 7) >> 3) * 8 * NT;
-  const int per = (U + 7) >> 3;
-  const int local = bid >> 3;
-  const int v = (bid & 7) * per + local;
-  if (local >= per || v >= U) return false;
-  const int tb = v / (8 * NT);
-  const int rem = v - tb * 8 * NT;
-  nt = rem >> 3;
-  const int tgi = tb * 8 + (rem & 7);
-  if (tgi >= n) return false;
+  int tgi;
+  if (!rows_unit_of(bid, n, NT, tgi, nt)) return false;
   te = a.tg[t0 + tgi];
   if (once)  // the expert's only group (an expert's groups are neighbours in the list)
     *once = (tgi == 0 || a.tg[t0 + tgi - 1].e != te.e) &&

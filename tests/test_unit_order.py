@@ -1,5 +1,6 @@
 """Work-group to unit arithmetic of the grouped GEMMs (exq_amd/csrc/unit_order.h), compiled for
-the CPU: the ranges of the combined tile launch as its kernel walks them."""
+the CPU: the ranges of the combined tile launch as its kernel walks them, and the order of the
+rows kernels' units."""
 import ctypes as C
 import subprocess
 from pathlib import Path
@@ -17,6 +18,9 @@ void t_mix(int t256, int t128, const int64_t* cap, int* tiles, int64_t* grid) {
   const MixTiles t = mix_tiles(t256, t128, cap[0], cap[1], cap[2], cap[3]);
   tiles[0] = t.ps; tiles[1] = t.i8; tiles[2] = t.t64; tiles[3] = t.bf;
   *grid = mix_grid(t, cap[0], cap[1], cap[2], cap[3]);
+}
+int t_rows_unit(int bid, int n, int n_tiles, int* tgi, int* nt) {
+  return rows_unit_of(bid, n, n_tiles, *tgi, *nt);
 }
 }
 """
@@ -64,3 +68,21 @@ def test_mix_ranges_hold_only_launched_tiles(lib, caps, groups, t256, t128):
         elif n:
             assert u > 0
     assert sum(units) <= grid, "the grid ends before the last unit"
+
+
+@pytest.mark.parametrize("n_tiles", [1, 3, 16, 224])
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 10, 11, 15, 16, 17, 24, 25, 31, 105])
+def test_rows_units_once_each_and_even_over_the_xcds(lib, n, n_tiles):
+    """Every unit is some work-group's (of a grid sized for n token groups or more), once, and no
+    XCD (work-group number modulo 8) has more than an eighth of them, rounded up."""
+    grid = 8 * -(-n // 8) * n_tiles
+    tgi, nt = C.c_int(), C.c_int()
+    seen, per_xcd = set(), [0] * 8
+    for bid in range(grid + 8 * n_tiles):
+        if lib.t_rows_unit(bid, n, n_tiles, C.byref(tgi), C.byref(nt)):
+            assert bid < grid
+            seen.add((tgi.value, nt.value))
+            per_xcd[bid % 8] += 1
+    assert seen == {(g, t) for g in range(n) for t in range(n_tiles)}
+    assert sum(per_xcd) == n * n_tiles
+    assert max(per_xcd) <= -(-n * n_tiles // 8)
