@@ -516,14 +516,21 @@ bool standard_shape(const exq_moe_problem* p) {
 // rows run on the rows kernels too (two launches fewer, no row sums, and half
 // the padding of 64-row groups): Qwen3 shape 64 x 256 tiles / rows kernels, us
 // per layer, T = 100 95 / 82, 187 122 / 111, 300 138 / 125, 500 (31 rows) 162 /
-// 161; OLMoE shape T = 187 136 / 115.
+// 161; OLMoE shape T = 187 136 / 115.  (All tokens on the same 8 of 128 experts, which
+// the host cannot see: T = 187 72 / 60, 300 75 / 78, 500 97 / 106.)
 bool rows_shape(const exq_moe_problem* p, bool mixed) {
   return !standard_shape(p) ||
          (!mixed && p->n_tokens * p->top_k <= kTokenGroupRows * p->n_experts);
 }
 
 // The unquantised GEMM takes the rows kernel up to this many rows per expert on
-// average.
+// average.  Whole call on cold weights, rows kernel / 128 x 128 tiles, us: 64 experts
+// of 2048 x 2048, 8 rows 134 / 169, 20 rows 138 / 172, 32 rows 181 / 177, Zipf ids
+// 175 / 204; 128 experts of 768 x 2048, 32 rows 125 / 130, Zipf 103 / 115; 8 experts
+// of 4096 x 4096, 32 rows 102 / 111.  Very large weights lose where experts pass 32
+// rows and win below (8 experts of 4096 x 28672: 28 rows each 318 / 387; Zipf ids
+// from 12 rows on 397 - 410 / 382 - 408; of 4096 x 14336 187 / 228 and 220 - 249 /
+// 224 - 238).
 constexpr int64_t kRowsBf16Max = 32;
 
 // ---- workspace layout of the fused forward --------------------------------------
