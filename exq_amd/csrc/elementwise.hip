@@ -95,50 +95,55 @@ __device__ __forceinline__ void store_vec(void* p, int64_t i, const float (&v)[V
 }
 
 // result[t, h] = sum_j w[t, j] * down[inv[t*k + j], h], j ascending, fp32.
-// One thread per VEC consecutive columns (8 with H % 8 == 0 and 16-byte aligned
-// rows, otherwise 1).  A token's positions, weights and rows are loaded SB slots
-// at a time, every load before its use, so eight slots are three dependent
-// round trips.  Bound: bytes; 2,648 rows of 2048 f16 values 9.4 -> 6.4 us
-// against one column per thread.
-constexpr int kCombineSlots = 8;
-
-template <int DT, int VEC>
+// Grid: tokens x column blocks; one thread per VEC consecutive columns (8 with
+// H % 8 == 0 and 16-byte aligned rows, otherwise 1).  A token's positions and
+// weights are scalar loads, and its rows go out SLOTS at a time.  Bound: bytes.
+// unsort_output of 24,576 bf16 rows in 4,096 tokens, against one column and one row
+// at a time: 2048 columns 82.3 -> 42.0 us, 2047 columns 82.6 -> 69.1 (93 with the
+// threads laid out over all outputs, whose 64-bit division found the token).
+template <int DT, int VEC, int SLOTS>
 __global__ void __launch_bounds__(256) combine_kernel(const void* __restrict__ down,
                                                       const int32_t* __restrict__ inv,
                                                       const void* __restrict__ w, int wdtype,
-                                                      int64_t n_units, int top_k, int H,
-                                                      int n_rows, void* __restrict__ out) {
-  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (u >= n_units) return;
-  const int per = H / VEC;
-  const int64_t t = u / per;
-  const int64_t h = (u - t * per) * VEC;
+                                                      int top_k, int H, int n_rows,
+                                                      void* __restrict__ out) {
+  const int64_t t = blockIdx.x;
+  const int64_t h = ((int64_t)blockIdx.y * blockDim.x + threadIdx.x) * VEC;
+  if (h >= H) return;
+  const int64_t slot0 = t * top_k;
   float acc[VEC];
 #pragma unroll
   for (int c = 0; c < VEC; ++c) acc[c] = 0.f;
-  for (int j0 = 0; j0 < top_k; j0 += kCombineSlots) {
-    int pos[kCombineSlots];
-    float wt[kCombineSlots], v[kCombineSlots][VEC];
+  for (int j0 = 0; j0 < top_k; j0 += SLOTS) {
+    int pos[SLOTS];
+    float wt[SLOTS], v[SLOTS][VEC];
 #pragma unroll
-    for (int j = 0; j < kCombineSlots; ++j) {
-      const bool in = j0 + j < top_k;
-      const int64_t slot = t * top_k + (in ? j0 + j : 0);
-      pos[j] = in ? inv[slot] : -1;
-      wt[j] = load_as_f32(w, wdtype, slot);
+    for (int j = 0; j < SLOTS; ++j)  // slots past the last repeat it, with weight 0
+      pos[j] = inv[slot0 + (j0 + j < top_k ? j0 + j : top_k - 1)];
+    if (wdtype == EXQ_DTYPE_F32) {
+      const float* wp = reinterpret_cast<const float*>(w) + slot0;
+#pragma unroll
+      for (int j = 0; j < SLOTS; ++j) wt[j] = wp[j0 + j < top_k ? j0 + j : top_k - 1];
+    } else {
+      const uint16_t* wp = reinterpret_cast<const uint16_t*>(w) + slot0;
+#pragma unroll
+      for (int j = 0; j < SLOTS; ++j) {
+        const uint32_t b = wp[j0 + j < top_k ? j0 + j : top_k - 1];
+        wt[j] = wdtype == EXQ_DTYPE_BF16 ? bf16_bits_to_f32(b) : f16_bits_to_f32(b);
+      }
     }
 #pragma unroll
-    for (int j = 0; j < kCombineSlots; ++j) {
+    for (int j = 0; j < SLOTS; ++j) {
       // (a position outside the rows: sort_order was not a permutation)
-      const bool ok = pos[j] >= 0 && pos[j] < n_rows;
-#pragma unroll
-      for (int c = 0; c < VEC; ++c) v[j][c] = 0.f;
-      if (ok) load_vec<DT, VEC>(down, (int64_t)pos[j] * H + h, v[j]);
+      const int row = (uint32_t)pos[j] < (uint32_t)n_rows ? pos[j] : 0;
+      load_vec<DT, VEC>(down, (int64_t)row * H + h, v[j]);
     }
 #pragma unroll
-    for (int j = 0; j < kCombineSlots; ++j) {
-      if (pos[j] < 0 || pos[j] >= n_rows) continue;
+    for (int j = 0; j < SLOTS; ++j) {
+      const bool use = j0 + j < top_k && (uint32_t)pos[j] < (uint32_t)n_rows;
+      const float wj = use ? wt[j] : 0.f;
 #pragma unroll
-      for (int c = 0; c < VEC; ++c) acc[c] += wt[j] * v[j][c];
+      for (int c = 0; c < VEC; ++c) acc[c] = fmaf(wj, use ? v[j][c] : 0.f, acc[c]);
     }
   }
   store_vec<DT, VEC>(out, t * H + h, acc);
@@ -264,19 +269,27 @@ static int launch_combine(const void* down_out, int dtype, const int32_t* inv, i
                           const void* router_weights, int weights_dtype, int64_t n_tokens,
                           int64_t top_k, int64_t hidden_size, void* result, hipStream_t s) {
   const bool vec = hidden_size % 8 == 0 && ((uintptr_t)down_out | (uintptr_t)result) % 16 == 0;
-  const int64_t units = n_tokens * (hidden_size / (vec ? 8 : 1));
-  EXQ_REQUIRE(cdiv(units, 256) <= INT32_MAX, "combine: too many outputs");
-  const dim3 grid((unsigned)cdiv(units, 256));
+  const int64_t cols = hidden_size / (vec ? 8 : 1), nby = cdiv(cols, 256);
+  const dim3 grid((unsigned)n_tokens, (unsigned)nby), block((unsigned)(64 * cdiv(cols, 64 * nby)));
+  auto launch = [&](auto dt, auto vc, auto slots) {
+    hipLaunchKernelGGL(
+        (combine_kernel<decltype(dt)::value, decltype(vc)::value, decltype(slots)::value>), grid,
+        block, 0, s, down_out, inv, router_weights, weights_dtype, (int)top_k, (int)hidden_size,
+        (int)n_active, result);
+  };
   with_dtype(dtype, [&](auto dt) {
-    constexpr int DT = decltype(dt)::value;
+    auto with_slots = [&](auto vc) {  // rows in flight: few spare loads in the last batch
+      if (top_k <= 2)
+        launch(dt, vc, std::integral_constant<int, 2>{});
+      else if (top_k <= 4 || cdiv(top_k, 4) % 2 == 1)
+        launch(dt, vc, std::integral_constant<int, 4>{});
+      else
+        launch(dt, vc, std::integral_constant<int, 8>{});
+    };
     if (vec)
-      hipLaunchKernelGGL((combine_kernel<DT, 8>), grid, dim3(256), 0, s, down_out, inv,
-                         router_weights, weights_dtype, units, (int)top_k, (int)hidden_size,
-                         (int)n_active, result);
+      with_slots(std::integral_constant<int, 8>{});
     else
-      hipLaunchKernelGGL((combine_kernel<DT, 1>), grid, dim3(256), 0, s, down_out, inv,
-                         router_weights, weights_dtype, units, (int)top_k, (int)hidden_size,
-                         (int)n_active, result);
+      with_slots(std::integral_constant<int, 1>{});
   });
   return check_launch("combine_kernel");
 }

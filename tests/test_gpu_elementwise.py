@@ -118,6 +118,48 @@ def test_combine_column_and_slot_edges(T, k, H, dtype, device):
     assert np.allclose(res.float().cpu().numpy(), ref, rtol=tol, atol=tol)
 
 
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 8, 12, 16])
+@pytest.mark.parametrize("H", [264, 257])
+@pytest.mark.parametrize("w_dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_combine_slot_batches(k, H, w_dtype, device):
+    """Slots in batches of 2, 4 and 8 with a short last one, in both column forms; a
+    NaN row reaches its own token alone."""
+    from exq_amd.kernels.exq_dispatch import combine
+    banner(f"combine batches k={k} H={H} {w_dtype}")
+    T = 13
+    rng = np.random.default_rng(k * 1000 + H)
+    down = torch.from_numpy(rng.standard_normal((T * k, H)).astype(np.float32))
+    w = torch.from_numpy(rng.random((T, k)).astype(np.float32)).to(w_dtype)
+    order = rng.permutation(T * k)
+    res = torch.empty(T, H, dtype=torch.float32, device=device)
+    ref = moe.combine(down.numpy(), order, w.float().numpy())
+    down[0] = float("nan")
+    combine(down.to(device), torch.from_numpy(order).to(device), w.to(device), res)
+    got = res.cpu().numpy()
+    own = order[0] // k
+    keep = np.arange(T) != own
+    # fp32 sums of k products of order 1: k ulp
+    assert np.allclose(got[keep], ref[keep], rtol=k * 2.4e-7, atol=k * 2.4e-7)
+    assert np.isnan(got[own]).all()
+
+
+def test_combine_past_2_32_outputs(device):
+    """More outputs than a launch has threads along one dimension."""
+    from exq_amd.kernels import unsort_output
+    T, N = (1 << 20) + 1, 4097
+    banner(f"unsort_output T={T} N={N}")
+    gen = torch.Generator(device=device).manual_seed(1)
+    ids = torch.randint(0, 4, (T, 1), generator=gen, device=device)
+    pos = torch.empty(T, dtype=torch.int64, device=device)
+    pos[torch.argsort(ids[:, 0], stable=True)] = torch.arange(T, device=device)
+    y = (torch.arange(T, device=device) % 251).to(torch.bfloat16)  # whole numbers: exact
+    w = torch.full((T, 1), 0.5, device=device)
+    out = unsort_output(y[:, None].expand(T, N).contiguous(), ids, w, 4)
+    want = (pos % 251).to(torch.bfloat16) * 0.5
+    assert all(bool((out[i:i + 65536] == want[i:i + 65536, None]).all())
+               for i in range(0, T, 65536))
+
+
 @pytest.mark.parametrize("rows,I", [(1, 8), (3, 12), (5, 1), (129, 2056)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_silu_and_mul_widths(rows, I, dtype, device):
