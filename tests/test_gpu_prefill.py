@@ -153,17 +153,19 @@ def test_prefill_per_expert_tile_shape_mixed_bank(act, device):
 
 
 def test_prefill_per_expert_tile_shape_none_big(device):
-    """A batch of 512 tokens (the per-expert switch is on) whose experts all stay
-    below 384 rows: the 128 x 256 range of the combined launch is empty and every
-    INT4 group takes the 64 x 256 tiles."""
+    """A batch of 600 tokens (the per-expert switch is on) whose experts all stay
+    below 384 rows and average more than 32 (fewer take the rows kernels): the
+    128 x 256 range of the combined launch is empty and every INT4 group takes the
+    64 x 256 tiles."""
     from exq_amd.kernels import fused_experts
     cfg = synth.MoeConfig("prefill_none_big", 52, 1024, 512, 32, 2, True, zipf=False)
-    T = 512
+    T = 600
     banner("prefill per-expert tile shape, no big expert")
     p13, s13, p2, s2 = _pack(cfg.n_experts, cfg.inter, cfg.hidden, 986, device)
     ids, w = synth.routing(cfg, T)
     counts = np.bincount(ids.reshape(-1), minlength=cfg.n_experts)
     assert counts.max() < 384 and T * cfg.top_k < 512 * cfg.n_experts
+    assert T >= 384 and T * cfg.top_k > 32 * cfg.n_experts
     x = _hidden(T, cfg.hidden, 987, device, torch.bfloat16)
     out = fused_experts(x, p13, s13, p2, s2, torch.from_numpy(w).to(device),
                         torch.from_numpy(ids).to(device))
@@ -320,15 +322,17 @@ def test_prefill_sorted_bf16_gemm_tiled(dtype, device):
     assert_close_rel(out, ref, TOL, f"grouped gemm tiled {dtype}")
 
 
-def test_prefill_mixed_mostly_int8_strided_grid(device):
-    """Mostly INT8 experts next to INT4 and BF16 ones at a large batch: the
-    grouped kernel's grid (capped while the tiled kernels run) strides over
-    more units than it has work-groups."""
+@pytest.mark.parametrize("H", [384, 512])
+def test_prefill_mixed_mostly_int8_strided_grid(H, device):
+    """Mostly INT8 experts next to INT4 and BF16 ones at a large batch.  H = 384,
+    which the 256-row tiles do not divide: they run on the grouped kernel, whose
+    grid (capped while the tiled kernels run) strides over more units than it has
+    work-groups.  H = 512: on the tiles."""
     from exq_amd.kernels import MixedExpertBank, fused_experts_mixed
-    banner("prefill mixed mostly int8")
+    banner(f"prefill mixed mostly int8 H={H}")
     T, E = 2000, 16
-    cfg = synth.MoeConfig("mix_int8", 46, 512, 512, E, 4, False)
-    w13, w2 = synth.expert_weights_gpu(E, 512, 512, 72, device)
+    cfg = synth.MoeConfig("mix_int8", 46, H, 512, E, 4, False)
+    w13, w2 = synth.expert_weights_gpu(E, 512, H, 72, device)
     tiers = [1] * E
     tiers[3] = 2
     tiers[9] = 0
@@ -336,20 +340,20 @@ def test_prefill_mixed_mostly_int8_strided_grid(device):
     ids, w = synth.routing(cfg, T)
     int8_rows = sum(int((ids == e).sum()) for e in range(E) if tiers[e] == 1)
     assert int8_rows // 64 * (512 // 16) > 2048  # more gate/up units than the capped grid
-    x = _hidden(T, 512, 950, device, torch.bfloat16)
+    x = _hidden(T, H, 950, device, torch.bfloat16)
     out = fused_experts_mixed(x, bank, torch.from_numpy(w).to(device),
                               torch.from_numpy(ids).to(device))
     from tests.test_gpu_mixed import _oracle
-    assert_close_rel(out, _oracle(bank, x, ids, w), TOL, "prefill mixed mostly int8")
+    assert_close_rel(out, _oracle(bank, x, ids, w), TOL, f"prefill mixed mostly int8 H={H}")
 
 
-@pytest.mark.parametrize("T", [300, 9000])
+@pytest.mark.parametrize("T", [300, 512, 513, 2000, 8192, 8193, 9000])
 def test_prefill_routing_plan_sizes(T, device):
-    """The fused layer's routing plan above one work-group: 2,400 slots take the
-    one-launch plan (every block recounts all slots), 72,000 slots the
-    three-launch plan through the workspace (per-block counts, offsets,
-    scatter).  sort_order / expert_ends are bit-exact; the output is within
-    0.5 % of the oracle on 64 sampled tokens."""
+    """The fused layer's routing plan: 2,400 and 4,096 slots in one work-group;
+    4,104, 16,000 and 65,536 in two launches (per-block counts, then places),
+    with ragged and whole last blocks; 65,544 and 72,000 in three through the
+    workspace (counts, offsets, scatter).  sort_order / expert_ends are
+    bit-exact; the output is within 0.5 % of the oracle on 64 sampled tokens."""
     from exq_amd.kernels import fused_experts
     cfg = synth.MoeConfig("plan_sizes", 48, 256, 128, 16, 8, True)
     banner(f"prefill routing plan T={T} ({T * cfg.top_k} slots)")
