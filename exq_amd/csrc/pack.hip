@@ -50,8 +50,9 @@ __device__ __forceinline__ void unpack8(const Raw8<DT>& r, float (&v)[8]) {
 // as IEEE division rounds it.  v * (1 / scale) is within 3 ulp of the quotient,
 // so both round to the same integer unless the product lies within TIE of a
 // half-way point (|v / scale| <= hi + 1, so 3 ulp are 1.5e-6 for INT4 and 2.4e-5
-// for INT8); only then, for one weight in 10^4 or fewer, the divisions are
-// done.  (A NaN product takes the first form; it is NaN in both.)
+// for INT8); only then the divisions are done.  That is 2 TIE of all weights, 2e-5
+// (INT4) and 2e-4 (INT8); a wave takes the branch when any of its 512 weights does,
+// 1 % and 10 % of them.  (A NaN product takes the first form; it is NaN in both.)
 template <int HI>
 __device__ __forceinline__ void quantize8(const float (&v)[8], float scale, int (&q)[8]) {
   constexpr float TIE = HI == 7 ? 1e-5f : 1e-4f;

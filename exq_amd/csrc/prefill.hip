@@ -1267,7 +1267,7 @@ __global__ void __launch_bounds__(TT, 2) tile_mix_kernel(GemmArgs a, TileArgs tp
                                                          TileArgs t64, TileArgs tbf) {
   static_assert(tile_a_stage<4, 4>() == AB_STAGE && tile_b_stage<4, 4>() == AB_STAGE &&
                     PS_A_STAGE == AB_STAGE && PS_B_STAGE == AB_STAGE,
-                "one LDS layout for the three tiles");
+                "one LDS layout for the four tiles");
   __shared__ __attribute__((aligned(1024))) unsigned char sA0[AB_STAGE];
   __shared__ __attribute__((aligned(1024))) unsigned char sA1[AB_STAGE];
   __shared__ __attribute__((aligned(1024))) unsigned char sB0[AB_STAGE];

@@ -116,6 +116,8 @@ __device__ void stable_scatter(int n, int nb, KeyFn key, int* run, uint32_t* mas
 // Past 4,096 items one work-group is too slow (8,000 items 21 us).
 constexpr int kSortTable = 2 * MASK_WORDS;  // (segment, bucket) counts, 16 bits each
 constexpr int kSortMax = 4096;              // items: four segments per wave
+// calls without a workspace for the block counts (route_plan_blocks) always fit
+static_assert((kRoutePlanOneBlock / 64) * MAX_BUCKETS <= kSortTable, "one work-group's table");
 
 // Whether n items over nb buckets fit one work-group.
 inline bool sort_fits(int64_t n, int64_t nb) {
