@@ -17,8 +17,9 @@
 // Bound.  With few rows per expert every weight is used once or twice, and a
 // chunk's copies, its dequantisation (14 VALU instructions per 8 weights) and
 // its LDS reads cost about the same.  Qwen3 shape at 187 tokens (105 token
-// groups), gate/up: 61 us; 39 us with only the copies left in, 46 us with only
-// the arithmetic.  Tiles of 16 or 64 rows, or of 256 weight rows, measured the
+// groups), gate/up: 52 us, the matrix pipes busy 15 % of it and 1.15 times the
+// weights fetched; when it took 61 us, 39 with only the copies left in and 46 with
+// only the arithmetic.  Tiles of 16 or 64 rows, or of 256 weight rows, measured the
 // same or slower there (109 - 123 us a layer against 111), and so did weights
 // copied two chunks at a time in whole 128-byte lines (113).  Three or four stages
 // instead of two, with three or two work-groups per CU: 95 -> 107 / 121 us (group
@@ -303,8 +304,10 @@ __device__ __forceinline__ void rows_body(const GemmArgs& a, int n_tiles,
   // at column s, dword kq of weight row brow(t) + r16.  Where a scale group holds
   // several steps (group 64, multiples of 128) the order of k inside it is free,
   // and a lane's weights for those steps are one read: k = 64 h + 16 kq + 8 j (step
-  // s = 2 h + j, 8 bytes) or k = 32 kq + 8 s (16 bytes), A read at the same k.  All
-  // these reads are free of bank conflicts under the maps above.  With the loop as
+  // s = 2 h + j, 8 bytes) or k = 32 kq + 8 s (16 bytes), A read at the same k.  These
+  // reads are free of bank conflicts under the maps above, but for group 64 outside
+  // gate/up: the 8-byte reads of a wave's two neighbouring weight tiles become one
+  // instruction there, 22 % of the LDS cycles conflicts.  With the loop as
   // one body per stage (fewer registers): Qwen3 shape at 187 tokens 98.4 -> 95.0 us
   // a layer, Mixtral at 100 tokens 315 -> 308, group 96 at 64 tokens 75 -> 70.5,
   // group 64 the same.
