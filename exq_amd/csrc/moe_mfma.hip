@@ -450,9 +450,9 @@ __global__ void __launch_bounds__(256) combine_partials_kernel(
       const int out_of = (int)(lo[q] | ((uint32_t)(E - 1) - lo[q]) | h32 | (0u - h32)) >> 31;
       const int shared = (k - 1 - j) >> 31, past = (kp - 1 - j) >> 31;
       const int drop = (out_of & ~shared) | past;
-      const int off = (q * H * 4 & ~drop) | (dev::OOB_OFF & drop);
-      pv[q] = __builtin_bit_cast(float4,
-                                 __builtin_amdgcn_raw_buffer_load_b128(rows, off + h * 4, 0, 0));
+      const uint32_t off = (q * H * 4 & ~drop) | (dev::OOB_OFF & drop);  // + h * 4 may pass 2^31
+      pv[q] = __builtin_bit_cast(
+          float4, __builtin_amdgcn_raw_buffer_load_b128(rows, (int)(off + (uint32_t)h * 4), 0, 0));
       wgt[q] = __int_as_float(((__float_as_int(wgt[q]) & ~shared) | (0x3f800000 & shared)) & ~drop);
     }
 #pragma unroll
